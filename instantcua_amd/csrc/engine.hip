@@ -174,8 +174,9 @@ struct icua_engine {
     bool persist_ok = false;
     // Matrix-core prefill buffers for chunks of up to pf_cap rows (allocated on first use).
     int pf_cap = 0;
-    float *px = nullptr, *pqkv = nullptr, *patt = nullptr, *ph = nullptr, *pxs = nullptr, *pts = nullptr;
-    uint16_t *pxa = nullptr, *pqh = nullptr, *pql = nullptr;
+    float *px = nullptr, *pqkv = nullptr, *patt = nullptr, *ph = nullptr, *pts = nullptr;
+    float *ppart = nullptr, *ppml = nullptr;  // K-split GEMM and key-split attention partials
+    uint16_t *pxa = nullptr, *pxb = nullptr, *pqh = nullptr, *pql = nullptr;
     // Vision tower, when the image holds it: weights, work buffers (one allocation, on first
     // use), the host copy of the position table, the prepared grid and the frame hash.
     uint8_t* d_vision = nullptr;
@@ -742,11 +743,11 @@ struct icua_engine {
     }
 
     void free_pf() {
-        void* bufs[] = {px, pqkv, patt, ph, pxs, pts, pxa, pqh, pql};
+        void* bufs[] = {px, pqkv, patt, ph, pts, pxa, pxb, pqh, pql, ppart, ppml};
         for (void* b : bufs)
             if (b) (void)hipFree(b);
-        px = pqkv = patt = ph = pxs = pts = nullptr;
-        pxa = pqh = pql = nullptr;
+        px = pqkv = patt = ph = pts = ppart = ppml = nullptr;
+        pxa = pxb = pqh = pql = nullptr;
         pf_cap = 0;
     }
 
@@ -760,7 +761,9 @@ struct icua_engine {
         HIPCK(hipMalloc(&patt, sizeof(float) * cap * H));
         HIPCK(hipMalloc(&ph, sizeof(float) * cap * FF));
         HIPCK(hipMalloc(&pxa, sizeof(uint16_t) * 2 * (size_t)cap * FF));
-        HIPCK(hipMalloc(&pxs, sizeof(float) * (size_t)cap * (FF / 64)));
+        HIPCK(hipMalloc(&pxb, sizeof(uint16_t) * (size_t)cap / 16 * (FF / 2048) * 2 * 512));
+        HIPCK(hipMalloc(&ppart, sizeof(float) * PF_PART_FLOATS));
+        HIPCK(hipMalloc(&ppml, sizeof(float) * PF_PART_ML_FLOATS));
         HIPCK(hipMalloc(&pts, sizeof(float) * (size_t)cap));
         HIPCK(hipMalloc(&pqh, sizeof(uint16_t) * (size_t)cap * NH * HD));
         HIPCK(hipMalloc(&pql, sizeof(uint16_t) * (size_t)cap * NH * HD));
@@ -771,58 +774,101 @@ struct icua_engine {
         return 0;
     }
 
+    // K-split partials of a residual GEMM (O, down) that the next reader of px adds to its rows.
+    struct PfPending {
+        int nsplit = 0;
+        const float* ds = nullptr;
+    };
+
     // One decoder layer over chunk rows [0, M) at cache slots p0.. (prompt rows row0..).
-    int enqueue_pf_layer(int l, int M, int Mpad, int p0, int row0, int vis_offset) {
+    int enqueue_pf_layer(int l, int M, int Mpad, int p0, int row0, int vis_offset, PfPending& pend) {
         const LayerW& w = L[l];
+        // fp16 operands: hi + lo parts (~22 bits), or with ICUA_FLAG_PREFILL_FP16 the hi part alone
+        // (fp16 activations, queries and probabilities: the reference engine's precision).
+        const int parts = (flags & ICUA_FLAG_PREFILL_FP16) ? 1 : 2;
         PfGemmArgs g{};
         g.xa = pxa;
-        g.xs = pxs;
+        g.xb = pxb;
         g.ts = pts;
         g.M = M;
         g.Mpad = Mpad;
         g.row0 = row0;
         g.vis_offset = vis_offset;
         g.n_vis = n_vis;
-        // fp16 operands: hi + lo parts (~22 bits), or with ICUA_FLAG_PREFILL_FP16 the hi part alone
-        // (fp16 activations, queries and probabilities: the reference engine's precision).
-        const int parts = (flags & ICUA_FLAG_PREFILL_FP16) ? 1 : 2;
         g.parts = parts;
+        g.part = ppart;
+        PfPrepArgs p = pf_prep_args(M, Mpad, row0, vis_offset);
+        p.parts = parts;
         // 1. RMSNorm + fused QKV.
-        HIPCK(launch_pf_prep(H, 1, px, w.attn_norm, M, Mpad, pxa, pxs, pts, parts, stream));
+        p.src = px;
+        p.norm_w = w.attn_norm;
+        p.nsplit = pend.nsplit;
+        p.ds = pend.ds;
+        HIPCK(launch_pf_prep(fmt, PF_SRC_RESID, p, stream));
         g.w = w.wqkv;
         g.sb = w.wqkv_sb;
         g.N = QKV;
         g.y = pqkv;
+        g.splits = pf_gemm_splits(fmt, H, QKV, M);
         HIPCK(launch_pf_gemm(fmt, H, EPI_STORE, g, stream));
         // 2. q/k norm + M-RoPE + KV write, causal flash attention.
         uint16_t* ql = parts == 2 ? pql : nullptr;
-        PfQkArgs qa{pqkv, w.q_norm, w.k_norm, rope, kv_ptr(l, 0), kv_ptr(l, 1), pqh, ql, M, p0, maxctx};
+        PfQkArgs qa{g.splits > 1 ? ppart : pqkv, w.q_norm, w.k_norm, rope, kv_ptr(l, 0), kv_ptr(l, 1), pqh, ql, M, p0,
+                    maxctx, g.splits};
         HIPCK(launch_pf_qk(qa, stream));
-        PfAttnArgs aa{pqh, ql, kv_ptr(l, 0), kv_ptr(l, 1), patt, M, p0, maxctx};
+        PfAttnArgs aa{pqh, ql, kv_ptr(l, 0), kv_ptr(l, 1), patt, M, p0, maxctx, pf_attn_splits(M, p0), ppart, ppml};
         HIPCK(launch_pf_attn(aa, stream));
         // 3. O projection + residual.
-        HIPCK(launch_pf_prep(H, 0, patt, nullptr, M, Mpad, pxa, pxs, pts, parts, stream));
+        p.src = patt;
+        p.nsplit = aa.nsplit;
+        p.ds = nullptr;
+        HIPCK(launch_pf_prep(fmt, PF_SRC_ATTN, p, stream));
         g.w = w.wo;
         g.sb = w.wo_sb;
         g.N = H;
         g.y = px;
+        g.splits = pf_gemm_splits(fmt, H, H, M);
         HIPCK(launch_pf_gemm(fmt, H, EPI_RESID, g, stream));
         // 4. RMSNorm + gate|up + SwiGLU.
-        HIPCK(launch_pf_prep(H, 1, px, w.mlp_norm, M, Mpad, pxa, pxs, pts, parts, stream));
+        p.src = px;
+        p.norm_w = w.mlp_norm;
+        p.nsplit = g.splits > 1 ? g.splits : 0;
+        HIPCK(launch_pf_prep(fmt, PF_SRC_RESID, p, stream));
         g.w = w.wgu;
         g.sb = w.wgu_sb;
         g.N = GU;
         g.h = ph;
+        g.splits = pf_gemm_splits(fmt, H, GU, M);
         HIPCK(launch_pf_gemm(fmt, H, EPI_SWIGLU, g, stream));
         // 5. Down projection + residual (+ DeepStack after layers 0-2 at visual rows).
-        HIPCK(launch_pf_prep(FF, 0, ph, nullptr, M, Mpad, pxa, pxs, pts, parts, stream));
+        p.src = ph;
+        p.nsplit = g.splits;
+        HIPCK(launch_pf_prep(fmt, PF_SRC_SWIGLU, p, stream));
         g.w = w.wd;
         g.sb = w.wd_sb;
         g.N = H;
         g.y = px;
         g.ds = (has_ds && l < 3) ? ds[l] : nullptr;
+        g.splits = pf_gemm_splits(fmt, FF, H, M);
         HIPCK(launch_pf_gemm(fmt, FF, EPI_RESID, g, stream));
+        pend = g.splits > 1 ? PfPending{g.splits, g.ds} : PfPending{};
         return 0;
+    }
+
+    PfPrepArgs pf_prep_args(int M, int Mpad, int row0, int vis_offset) const {
+        PfPrepArgs p{};
+        p.dst = px;
+        p.M = M;
+        p.Mpad = Mpad;
+        p.xa = pxa;
+        p.xb = pxb;
+        p.ts = pts;
+        p.part = ppart;
+        p.part_ml = ppml;
+        p.row0 = row0;
+        p.vis_offset = vis_offset;
+        p.n_vis = n_vis;
+        return p;
     }
 
     // Matrix-core prefill of prompt rows [0, n) at slots start_pos.., then the last row's
@@ -832,7 +878,7 @@ struct icua_engine {
         int M = 0;
         for (int c0 = 0; c0 < n; c0 += PF_CHUNK) {
             M = std::min(PF_CHUNK, n - c0);
-            const int Mpad = (M + 127) / 128 * 128;
+            const int pad = pf_use_split(M) ? 64 : 128, Mpad = (M + pad - 1) / pad * pad;
             EmbedArgs ea{};
             ea.toks = prompt;
             ea.E = E;
@@ -844,10 +890,21 @@ struct icua_engine {
             ea.st = st;
             ea.n = M;
             HIPCK(launch_embed(ea, stream));
+            PfPending pend;
             for (int l = 0; l < layers; ++l)
-                if (enqueue_pf_layer(l, M, Mpad, start_pos + c0, c0, vis_offset)) return -1;
+                if (enqueue_pf_layer(l, M, Mpad, start_pos + c0, c0, vis_offset, pend)) return -1;
+            if (c0 + M < n) continue;
+            if (pend.nsplit) {
+                PfPrepArgs p = pf_prep_args(M, Mpad, c0, vis_offset);
+                p.src = px;
+                p.dst = x;
+                p.nsplit = pend.nsplit;
+                p.ds = pend.ds;
+                HIPCK(launch_pf_last_row(p, M - 1, stream));
+            } else {
+                HIPCK(hipMemcpyAsync(x, px + (size_t)(M - 1) * H, sizeof(float) * H, hipMemcpyDeviceToDevice, stream));
+            }
         }
-        HIPCK(hipMemcpyAsync(x, px + (size_t)(M - 1) * H, sizeof(float) * H, hipMemcpyDeviceToDevice, stream));
         HIPCK(launch_set_pass(st, start_pos + n - 1, 1, write_logits ? 1 : 0, stream));
         return enqueue_head(MAXM, 0);
     }

@@ -103,16 +103,35 @@ hipError_t launch_embed(const EmbedArgs& a, hipStream_t s);
 // Sets pos / n / logits_rows of the control block on the stream.
 hipError_t launch_set_pass(State* st, int pos, int n, int logits_rows, hipStream_t s);
 
-// ---- Matrix-core prefill (prefill.hip), q4 weights, passes of M <= Mpad tokens (Mpad % 128 == 0).
-// Activation operands of one GEMM input: fp16 hi / lo parts of the row-scaled activations
-// [Mpad / 16][K / 32][parts][64][8] (parts 2: hi and lo; 1: hi alone), group sums
-// [Mpad / 16][K / 64][16] and row scales [Mpad].
-hipError_t launch_pf_prep(int K, int norm, const float* src, const float* norm_w, int M, int Mpad, uint16_t* xa,
-                          float* xs, float* ts, int parts, hipStream_t s);
+// ---- Matrix-core prefill (prefill.hip), passes of M tokens.
+// Operand prep of one GEMM input of K = 2048 (PF_SRC_RESID, normalised; PF_SRC_ATTN) or 6144
+// (PF_SRC_SWIGLU): fp16 hi / lo parts of the row-scaled activations, q4 group-sum operands, row
+// scales (layouts in prefill.hip), rows M .. Mpad - 1 zero.
+enum PfSource { PF_SRC_RESID = 0, PF_SRC_ATTN = 1, PF_SRC_SWIGLU = 2 };
+struct PfPrepArgs {
+    const float* src;       // rows [M][K]
+    float* dst;             // PF_SRC_RESID with partials: where the summed residual rows go
+    const float* norm_w;    // PF_SRC_RESID
+    int M, Mpad, parts;     // parts 2: hi and lo; 1: hi alone
+    uint16_t* xa;           // [Mpad / 16][K / 32][parts][64][8]
+    uint16_t* xb;           // [Mpad / 16][ceil(K / 2048)][2][64][8] (q4, parts 2)
+    float* ts;              // [Mpad]
+    // K-split partials of the GEMM before, [nsplit][M][N]: PF_SRC_RESID (N = 2048) adds them to
+    // src when nsplit > 0; PF_SRC_SWIGLU (N = 12288) takes them in place of src when nsplit > 1;
+    // PF_SRC_ATTN takes the attention's key-split partials (PfAttnArgs) when nsplit > 1.
+    const float* part;
+    const float* part_ml;
+    int nsplit;
+    const float* ds;        // PF_SRC_RESID: DeepStack rows [n_vis][H] to add or null
+    int row0, vis_offset, n_vis;
+};
+hipError_t launch_pf_prep(int fmt, int src, const PfPrepArgs& a, hipStream_t s);
+// Residual row t with the pending partials added, to dst [H].
+hipError_t launch_pf_last_row(const PfPrepArgs& a, int t, hipStream_t s);
 
 struct PfGemmArgs {
     const uint16_t* xa;     // activation operands (launch_pf_prep)
-    const float* xs;        // group sums
+    const uint16_t* xb;     // q4 group-sum operands
     const float* ts;        // row scales
     const uint8_t* w;       // codes in 16-row MFMA tiles (launch_repack)
     const uint8_t* sb;      // q4 half2 (scale, bias) [N][K / 64]; q8 half scales [N][K / 32]
@@ -123,13 +142,24 @@ struct PfGemmArgs {
     int row0;               // prompt row of pass row 0
     int vis_offset, n_vis;
     int parts;              // operand parts of xa (1 or 2, as launch_pf_prep wrote them)
+    int splits;             // pf_gemm_splits(): > 1 stores K-split partials [splits][M][N] to part
+    float* part;
 };
+// Prompts of up to PF_SPLIT_M rows take the K-split GEMM.
+constexpr int PF_SPLIT_M = 1024;
+inline bool pf_use_split(int M) { return M <= PF_SPLIT_M; }
+int pf_gemm_splits(int fmt, int K, int N, int M);
+// Partials of a GEMM (at most 256 tiles of 64 x 256) or an attention (256 / 8 query
+// blocks and splits of 64 rows), floats.
+constexpr size_t PF_PART_FLOATS = (size_t)256 * 64 * 256;
+constexpr size_t PF_PART_ML_FLOATS = (size_t)32 * 64 * NH * 2;
+static_assert(PF_PART_FLOATS >= (size_t)32 * 64 * H, "attention partials");
 // fmt: FMT_Q4 / FMT_Q8 / FMT_F16 (sb unused for f16); epi: EPI_STORE / EPI_RESID / EPI_SWIGLU;
 // K = 2048 (any epilogue) or 6144 (EPI_RESID).
 hipError_t launch_pf_gemm(int fmt, int K, int epi, const PfGemmArgs& a, hipStream_t s);
 
 struct PfQkArgs {
-    const float* qkv;       // raw fused QKV rows [M][QKV]
+    const float* qkv;       // raw fused QKV rows [M][QKV], or nsplit partials of them [nsplit][M][QKV]
     const float* q_norm;
     const float* k_norm;
     const float* rope;      // [maxctx][64] (cos, sin)
@@ -138,6 +168,7 @@ struct PfQkArgs {
     uint16_t* qh;           // queries, pre-scaled, fp16 hi / lo parts [Mpad][NH][HD]
     uint16_t* ql;
     int M, p0, maxctx;      // rows of the pass at cache slots p0 .. p0 + M - 1
+    int nsplit;
 };
 hipError_t launch_pf_qk(const PfQkArgs& a, hipStream_t s);
 
@@ -148,7 +179,11 @@ struct PfAttnArgs {
     const uint16_t* vc;
     float* out;             // attention rows [M][H] fp32
     int M, p0, maxctx;
+    int nsplit;             // pf_attn_splits(): > 1 stores unnormalised rows [nsplit][M][H] to part
+    float* part;            // and (max, denominator) pairs [nsplit][M][NH] to part_ml
+    float* part_ml;
 };
+int pf_attn_splits(int M, int p0);
 hipError_t launch_pf_attn(const PfAttnArgs& a, hipStream_t s);
 
 // Bit-exact dequantisation of rows [row0, row0 + rows) to fp32 (w = s*q + b / s*q / half),

@@ -24,6 +24,8 @@
 // fp32 queries and probabilities are split into fp16 hi + lo parts (two products each), which
 // keeps them at ~22 bits against the fp16 cache (one part with fp16 operands alone).  Each wave
 // holds 32 queries, so every K and V operand it reads from LDS feeds two products.
+#include <algorithm>
+
 #include "icua_device.h"
 #include "icua_kernels.h"
 
@@ -32,37 +34,106 @@ namespace icua {
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 typedef _Float16 v4h __attribute__((ext_vector_type(4)));
 
-// ------------------------------------------------------------------------------------------
-// Activation operands.  XA: [Mpad / 16][K / 32][2 (hi, lo)][64 lanes][8 halves], lane l
-// holding token 16 tb + l % 16, K = 32 ks + 8 (l / 16) + 0..7.  XS: [Mpad / 16][K / 64][16]
-// group sums of hi + lo.  TS: [Mpad] row scales 2^(E_t - 14).  One workgroup per token row
-// (rows >= M are zero).  A row writes 16-byte pieces of lines that the 16 rows of its token
-// block share, so rows are dealt to the 8 XCDs (workgroup i runs on XCD i % 8) in contiguous
-// ranges: the lines are completed in one L2 rather than written back in parts from eight.
+__device__ __forceinline__ float swiglu(float y, float up) {
+    return y * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-y * 1.4426950408889634f)) * up;
+}
 
-template <int K, bool NORM, int HL>
-__global__ __launch_bounds__(256) void pf_prep_kernel(const float* __restrict__ src, const float* __restrict__ norm_w,
-                                                      int M, uint16_t* __restrict__ xa, float* __restrict__ xs,
-                                                      float* __restrict__ ts) {
+// ------------------------------------------------------------------------------------------
+// Activation operands.  XA: [Mpad / 16][K / 32][parts (hi, lo)][64 lanes][8 halves], lane l
+// holding token 16 tb + l % 16.  q8 / f16: K = 32 ks + 8 (l / 16) + 0..7 of k-step ks, in order.
+// q4 takes the K order in which its nibbles unpack without cross-lane moves: k-step 2 g + h of
+// 64-group g holds K = 64 g + 16 (l / 16) + 8 h + {0, 2, 4, 6, 1, 3, 5, 7}.  XB (q4, hi + lo):
+// the 64-group sums of hi + lo times 2^-8 (into fp16 range), as fp16 hi and lo A operands over
+// groups, [Mpad / 16][ceil(K / 2048)][2][64 lanes][8].  TS: [Mpad] row scales 2^(E_t - 14).  One
+// workgroup per token row (rows >= M are zero).  A row writes 16-byte pieces of lines that the 16
+// rows of its token block share, so rows are dealt to the 8 XCDs (workgroup i runs on XCD i % 8)
+// in contiguous ranges: the lines are completed in one L2 rather than written back in parts.
+//
+// The source row is what the previous kernel left, so that no pass over memory only moves data:
+// a residual row, to which the O / down GEMM's K-split partial sums (and DeepStack rows) are
+// added and written back; attention rows, or their key-split partials, merged; SwiGLU rows, or
+// the gate|up GEMM's K-split partials.
+template <int K, int SRC, int HL, bool Q4>
+__global__ __launch_bounds__(256) void pf_prep_kernel(PfPrepArgs a) {
     constexpr int NU = K / 8 / 256;  // units of 8 activations per thread
-    constexpr int NG = K / 64, NKS = K / 32;
+    constexpr int NKS = K / 32, NXB = (K / 64 + 31) / 32;
     const int t = (int)(blockIdx.x % 8) * (int)(gridDim.x / 8) + (int)(blockIdx.x / 8);  // gridDim.x % 8 == 0
     const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
     __shared__ float red[8];
     float v[NU][8];
+    auto add8 = [](float(&d)[8], const float* p) {
+        const float4 a0 = ((const float4*)p)[0], a1 = ((const float4*)p)[1];
+        d[0] += a0.x; d[1] += a0.y; d[2] += a0.z; d[3] += a0.w;
+        d[4] += a1.x; d[5] += a1.y; d[6] += a1.z; d[7] += a1.w;
+    };
 #pragma unroll
-    for (int j = 0; j < NU; ++j) {
-        if (t < M) {
-            const float4* p = (const float4*)(src + (size_t)t * K + (tid + 256 * j) * 8);
-            const float4 a0 = p[0], a1 = p[1];
-            v[j][0] = a0.x; v[j][1] = a0.y; v[j][2] = a0.z; v[j][3] = a0.w;
-            v[j][4] = a1.x; v[j][5] = a1.y; v[j][6] = a1.z; v[j][7] = a1.w;
+    for (int j = 0; j < NU; ++j)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[j][i] = 0.f;
+    float4 w0, w1;  // requested with the row, not after its sum of squares
+    if constexpr (SRC == PF_SRC_RESID) {
+        static_assert(SRC != PF_SRC_RESID || NU == 1, "one unit per thread");
+        w0 = ((const float4*)(a.norm_w + tid * 8))[0];
+        w1 = ((const float4*)(a.norm_w + tid * 8))[1];
+    }
+    if (t < a.M) {
+        if (SRC == PF_SRC_ATTN && a.nsplit > 1) {
+            // Merge of the attention's key splits: head tid / 16, dims 8 (tid % 16) .. + 7.
+            const int head = tid >> 4;
+            const float2* ml = (const float2*)a.part_ml + (size_t)t * NH + head;
+            const size_t mls = (size_t)a.M * NH, os = (size_t)a.M * H;
+            const float* op = a.part + (size_t)t * H + 8 * tid;
+            float m = -__builtin_inff();
+            for (int s = 0; s < a.nsplit; ++s) m = fmaxf(m, ml[s * mls].x);  // finite: each row sees its own key
+            float l = 0.f;
+#pragma unroll 4
+            for (int s = 0; s < a.nsplit; ++s) {
+                const float2 x = ml[s * mls];
+                const float f = x.x == -__builtin_inff() ? 0.f : __builtin_amdgcn_exp2f(x.x - m);
+                const float4 a0 = ((const float4*)(op + s * os))[0], a1 = ((const float4*)(op + s * os))[1];
+                l = fmaf(x.y, f, l);
+                v[0][0] = fmaf(a0.x, f, v[0][0]); v[0][1] = fmaf(a0.y, f, v[0][1]);
+                v[0][2] = fmaf(a0.z, f, v[0][2]); v[0][3] = fmaf(a0.w, f, v[0][3]);
+                v[0][4] = fmaf(a1.x, f, v[0][4]); v[0][5] = fmaf(a1.y, f, v[0][5]);
+                v[0][6] = fmaf(a1.z, f, v[0][6]); v[0][7] = fmaf(a1.w, f, v[0][7]);
+            }
+            const float inv = 1.0f / l;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) v[0][i] *= inv;
+        } else if (SRC == PF_SRC_SWIGLU && a.nsplit > 1) {
+            // Units 8 u .. + 7 are row block u of the gate|up GEMM: 8 gate rows, then 8 up rows.
+#pragma unroll
+            for (int j = 0; j < NU; ++j) {
+                float up[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+                const float* p = a.part + (size_t)t * GU + (size_t)(tid + 256 * j) * 16;
+                for (int s = 0; s < a.nsplit; ++s) {
+                    add8(v[j], p + (size_t)s * a.M * GU);
+                    add8(up, p + (size_t)s * a.M * GU + 8);
+                }
+#pragma unroll
+                for (int i = 0; i < 8; ++i) v[j][i] = swiglu(v[j][i], up[i]);
+            }
         } else {
 #pragma unroll
-            for (int i = 0; i < 8; ++i) v[j][i] = 0.f;
+            for (int j = 0; j < NU; ++j) add8(v[j], a.src + (size_t)t * K + (tid + 256 * j) * 8);
+            if (SRC == PF_SRC_RESID && a.nsplit > 0) {
+                const float* p = a.part + (size_t)t * H + tid * 8;
+                float y[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+                for (int s = 0; s < a.nsplit; ++s) add8(y, p + (size_t)s * a.M * H);
+#pragma unroll
+                for (int i = 0; i < 8; ++i) v[0][i] += y[i];
+                if (a.ds) {  // DeepStack residual of a visual row (Shaders.swift:696-707)
+                    const int vrow = a.row0 + t - a.vis_offset;
+                    if (a.vis_offset >= 0 && vrow >= 0 && vrow < a.n_vis) add8(v[0], a.ds + (size_t)vrow * H + tid * 8);
+                }
+                float4* xo = (float4*)(a.dst + (size_t)t * K + tid * 8);
+                xo[0] = make_float4(v[0][0], v[0][1], v[0][2], v[0][3]);
+                xo[1] = make_float4(v[0][4], v[0][5], v[0][6], v[0][7]);
+            }
         }
     }
-    if constexpr (NORM) {
+    if constexpr (SRC == PF_SRC_RESID) {
         float ss = 0.f;
 #pragma unroll
         for (int j = 0; j < NU; ++j)
@@ -73,14 +144,9 @@ __global__ __launch_bounds__(256) void pf_prep_kernel(const float* __restrict__ 
         __syncthreads();
         const float tot = (red[0] + red[1]) + (red[2] + red[3]);
         const float scale = 1.0f / sqrtf(tot / (float)K + EPS);
+        const float w[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
 #pragma unroll
-        for (int j = 0; j < NU; ++j) {
-            const float4* wp = (const float4*)(norm_w + (tid + 256 * j) * 8);
-            const float4 w0 = wp[0], w1 = wp[1];
-            const float w[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
-#pragma unroll
-            for (int i = 0; i < 8; ++i) v[j][i] = v[j][i] * scale * w[i];
-        }
+        for (int i = 0; i < 8; ++i) v[0][i] = v[0][i] * scale * w[i];
     }
     // Row exponent: largest |x| in [2^E, 2^(E+1)).
     float amax = 0.f;
@@ -102,27 +168,100 @@ __global__ __launch_bounds__(256) void pf_prep_kernel(const float* __restrict__ 
         float gs = 0.f;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const float x0 = ldexpf(v[j][2 * i], sh), x1 = ldexpf(v[j][2 * i + 1], sh);
+            // Word i holds K 2 i, 2 i + 1, or in q4 order (0, 2) (4, 6) (1, 3) (5, 7).
+            const int i0 = Q4 ? 4 * (i & 1) + (i >> 1) : 2 * i, i1 = Q4 ? i0 + 2 : i0 + 1;
+            const float x0 = ldexpf(v[j][i0], sh), x1 = ldexpf(v[j][i1], sh);
             const f16 h0 = (f16)x0, h1 = (f16)x1;
             const f16 l0 = (f16)(x0 - (float)h0), l1 = (f16)(x1 - (float)h1);
-            if constexpr (HL == 2)
-                gs += ((float)h0 + (float)l0) + ((float)h1 + (float)l1);
-            else
-                gs += (float)h0 + (float)h1;
+            gs += ((float)h0 + (float)l0) + ((float)h1 + (float)l1);
             hw[i] = (uint32_t)__builtin_bit_cast(uint16_t, h0) | ((uint32_t)__builtin_bit_cast(uint16_t, h1) << 16);
             lw[i] = (uint32_t)__builtin_bit_cast(uint16_t, l0) | ((uint32_t)__builtin_bit_cast(uint16_t, l1) << 16);
         }
-        // Group sums over the 8 adjacent lanes holding the group's 64 values.
-        gs += dpp<DPP_XOR1>(gs);
-        gs += dpp<DPP_XOR2>(gs);
-        gs += dpp<DPP_HALF_MIRROR>(gs);
-        const int ks = k0 / 32, qq = (k0 % 32) / 8;
-        uint16_t* base = xa + ((size_t)(tb * NKS + ks) * HL) * 512 + (tr + 16 * qq) * 8;
+        const int ks = Q4 ? 2 * (k0 / 64) + (k0 % 16) / 8 : k0 / 32, qq = Q4 ? (k0 % 64) / 16 : (k0 % 32) / 8;
+        uint16_t* base = a.xa + ((size_t)(tb * NKS + ks) * HL) * 512 + (tr + 16 * qq) * 8;
         *(uint4*)base = make_uint4(hw[0], hw[1], hw[2], hw[3]);
         if constexpr (HL == 2) *(uint4*)(base + 512) = make_uint4(lw[0], lw[1], lw[2], lw[3]);
-        if (k0 % 64 == 0) xs[(size_t)(tb * NG + k0 / 64) * 16 + tr] = gs;
+        if constexpr (Q4 && HL == 2) {
+            // Group sums over the 8 adjacent lanes holding the group's 64 values.
+            gs += dpp<DPP_XOR1>(gs);
+            gs += dpp<DPP_XOR2>(gs);
+            gs += dpp<DPP_HALF_MIRROR>(gs);
+            if (k0 % 64 == 0) {
+                const int g = k0 / 64;
+                const float x = gs * 0.00390625f;  // 2^-8: a group sum of 64 values below 2^15
+                const f16 hx = (f16)x;
+                uint16_t* xb = a.xb + ((size_t)(tb * NXB + g / 32) * 2 * 64 + tr + 16 * ((g % 32) / 8)) * 8 + g % 8;
+                xb[0] = __builtin_bit_cast(uint16_t, hx);
+                xb[512] = f2h(x - (float)hx);
+            }
+        }
     }
-    if (tid == 0) ts[t] = ldexpf(1.0f, -sh);
+    if (tid == 0) a.ts[t] = ldexpf(1.0f, -sh);
+}
+
+// The residual row t0 after a GEMM that left K-split partials: dst = src + partials (+ DeepStack).
+__global__ __launch_bounds__(256) void pf_last_row_kernel(PfPrepArgs a, int t) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    float y = 0.f;
+    for (int s = 0; s < a.nsplit; ++s) y += a.part[((size_t)s * a.M + t) * H + i];
+    float v = a.src[(size_t)t * H + i] + y;
+    const int vrow = a.row0 + t - a.vis_offset;
+    if (a.ds && a.vis_offset >= 0 && vrow >= 0 && vrow < a.n_vis) v += a.ds[(size_t)vrow * H + i];
+    a.dst[i] = v;
+}
+
+// ------------------------------------------------------------------------------------------
+// Weight codes as fp16 B operands, exactly.
+
+// Eight q4 codes of a dword (byte j: K j low, K 4 + j high): a nibble or'ed into 0x6400 is the
+// fp16 value 1024 + q (or 1024 + 16 q in place of the high nibble), and one packed operation
+// leaves q.  Halves in K order 0, 2, 4, 6, 1, 3, 5, 7.
+__device__ __forceinline__ uint32_t and_or(uint32_t d, uint32_t mask, uint32_t bits) {
+    uint32_t r;  // one instruction (from two literals the compiler makes two)
+    asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(d), "s"(mask), "v"(bits));
+    return r;
+}
+__device__ __forceinline__ void unpack_q4(uint32_t d, f16x2 (&o)[4]) {
+    const f16x2 k1024 = {(f16)1024.f, (f16)1024.f}, k16 = {(f16)0.0625f, (f16)0.0625f}, k64 = {(f16)-64.f, (f16)-64.f};
+    const uint32_t e = d >> 8;
+    o[0] = as_h2(and_or(d, 0x000F000Fu, 0x64006400u)) - k1024;
+    o[1] = __builtin_elementwise_fma(as_h2(and_or(d, 0x00F000F0u, 0x64006400u)), k16, k64);
+    o[2] = as_h2(and_or(e, 0x000F000Fu, 0x64006400u)) - k1024;
+    o[3] = __builtin_elementwise_fma(as_h2(and_or(e, 0x00F000F0u, 0x64006400u)), k16, k64);
+}
+// Eight q8 codes of two dwords in order: a signed byte with its top bit flipped, put under the
+// exponent of 1024 by a byte permute, is the fp16 value 1152 + b.
+__device__ __forceinline__ void unpack_q8(uint32_t d0, uint32_t d1, f16x2 (&o)[4]) {
+    const f16x2 k1152 = {(f16)1152.f, (f16)1152.f};
+    const uint32_t u0 = d0 ^ 0x80808080u, u1 = d1 ^ 0x80808080u;
+    o[0] = as_h2(__builtin_amdgcn_perm(0x64646464u, u0, 0x04010400u)) - k1152;
+    o[1] = as_h2(__builtin_amdgcn_perm(0x64646464u, u0, 0x04030402u)) - k1152;
+    o[2] = as_h2(__builtin_amdgcn_perm(0x64646464u, u1, 0x04010400u)) - k1152;
+    o[3] = as_h2(__builtin_amdgcn_perm(0x64646464u, u1, 0x04030402u)) - k1152;
+}
+__device__ __forceinline__ uint4 pack4(const f16x2 (&o)[4]) {
+    return make_uint4(h2_bits(o[0]), h2_bits(o[1]), h2_bits(o[2]), h2_bits(o[3]));
+}
+
+// One output of a GEMM tile: token t of weight row `row` (y with the row scale applied).
+template <int EPI>
+__device__ __forceinline__ void pf_store(const PfGemmArgs& a, int t, int row, float y) {
+    if constexpr (EPI == EPI_STORE) {
+        if (t < a.M) a.y[(size_t)t * a.N + row] = y;
+    } else if constexpr (EPI == EPI_RESID) {
+        if (t < a.M) {
+            float* xo = a.y + (size_t)t * a.N + row;
+            float v = *xo + y;
+            if (a.ds) {  // DeepStack residual of a visual row (Shaders.swift:696-707)
+                const int vrow = a.row0 + t - a.vis_offset;
+                if (a.vis_offset >= 0 && vrow >= 0 && vrow < a.n_vis) v = v + a.ds[(size_t)vrow * H + row];
+            }
+            *xo = v;
+        }
+    } else {  // EPI_SWIGLU: a row block holds 8 gate units, then their up rows (lanes r16, r16 ^ 8)
+        const float up = dpp<0x128>(y);  // lane r16 ^ 8 of the row of 16 (a rotation by 8)
+        if (t < a.M && (row & 15) < 8) a.h[(size_t)t * FF + (row >> 4) * 8 + (row & 15)] = swiglu(y, up);
+    }
 }
 
 // ------------------------------------------------------------------------------------------
@@ -211,83 +350,49 @@ __global__ __launch_bounds__(512) void pf_gemm_kernel(PfGemmArgs a) {
                 for (int j = 0; j < 2; ++j) Dn[hb][j] = dsrc[hb * DSRC2 + 2 * c + j];
         }
     };
-    // Nibble lane L (row L % 16, 16-K slot L / 16 of each group) -> fp16 lanes (L % 16) + 16 (2 (slot % 2) + h)
-    // of k-step 2 gg + slot / 2, h = 0 for K 0..7 of the slot, 1 for K 8..15.
+    // A chunk's lane is the B-operand lane of every format (XA follows the q4 K order).
     auto lstore = [&](int b) {
 #pragma unroll
-      for (int hb = 0; hb < NHF; ++hb) {
-        const int sr = srb + 8 * hb;
-        if constexpr (FMT == FMT_F16) {
-            // f16 chunk j is k-step j, already in the B-operand lane layout.
+        for (int hb = 0; hb < NHF; ++hb) {
+            const int sr = srb + 8 * hb;
+            if constexpr (FMT == FMT_F16) {  // chunk j is k-step j
 #pragma unroll
-            for (int j = 0; j < 4; ++j) Bs[b][sr][j][lane] = Wn[hb][j];
-            continue;
-        } else if constexpr (FMT == FMT_Q8) {
-            // q8 chunk j: bytes 0-7 of a lane are k-step 2 j (K-slot lane / 16 of row lane % 16),
-            // bytes 8-15 k-step 2 j + 1, the B-operand lane layout; a signed byte b spread into a
-            // 16-bit lane, xor 0x80 and or'ed into 0x6400, is the fp16 value 1152 + b, and one
-            // packed fp16 subtraction leaves b exactly.
-            const f16x2 k1152 = {(f16)1152.f, (f16)1152.f};
-#pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                const uint32_t dd[4] = {Wn[hb][j].x, Wn[hb][j].y, Wn[hb][j].z, Wn[hb][j].w};
-#pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    uint32_t o[4];
-                    // DQ: k-step 2 j + h is 32-group 4 c + 2 j + h, the scale in half h of word 2 c + j.
-                    const f16 sc = DQ ? (h ? as_h2(Dn[hb][j]).y : as_h2(Dn[hb][j]).x) : (f16)1.f;
-                    const f16x2 sc2 = {sc, sc};
-#pragma unroll
-                    for (int w2 = 0; w2 < 2; ++w2) {
-                        const uint32_t d = dd[2 * h + w2];
-                        const uint32_t s0 = __builtin_amdgcn_perm(d, d, 0x0C010C00u);  // b0, b1
-                        const uint32_t s1 = __builtin_amdgcn_perm(d, d, 0x0C030C02u);  // b2, b3
-                        f16x2 q0 = as_h2((s0 ^ 0x00800080u) | 0x64006400u) - k1152;
-                        f16x2 q1 = as_h2((s1 ^ 0x00800080u) | 0x64006400u) - k1152;
-                        if constexpr (DQ) {
-                            q0 = q0 * sc2;
-                            q1 = q1 * sc2;
-                        }
-                        o[2 * w2] = h2_bits(q0);
-                        o[2 * w2 + 1] = h2_bits(q1);
-                    }
-                    Bs[b][sr][2 * j + h][lane] = make_uint4(o[0], o[1], o[2], o[3]);
-                }
-            }
-            continue;
-        } else {
-        const int r = lane & 15, slot = lane >> 4;
-        const uint32_t dd[4] = {Wn[hb][0].x, Wn[hb][0].y, Wn[hb][0].z, Wn[hb][0].w};
-#pragma unroll
-        for (int gg = 0; gg < 2; ++gg) {
-            // DQ: 64-group 2 c + gg of this row, (scale, bias) in word 2 c + gg.
-            const f16x2 sbw = as_h2(DQ ? Dn[hb][gg] : 0x00003C00u);
-            const f16x2 sc2 = {sbw.x, sbw.x}, bi2 = {sbw.y, sbw.y};
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const uint32_t d = dd[2 * gg + h];
-                uint32_t o[4];
+                for (int j = 0; j < 4; ++j) Bs[b][sr][j][lane] = Wn[hb][j];
+            } else if constexpr (FMT == FMT_Q8) {
+                // Bytes 0-7 of a lane of chunk j are k-step 2 j, bytes 8-15 k-step 2 j + 1.
 #pragma unroll
                 for (int j = 0; j < 2; ++j) {
-                    // K 8 h + 2 j, + 1 are the low nibbles of bytes 2 j, 2 j + 1; K 8 h + 4 + 2 j, + 1 the
-                    // high ones.  Bytes spread to 16-bit lanes, a nibble or'ed into 0x6400 is the fp16
-                    // value 1024 + q, and one packed fp16 subtraction leaves q exactly.
-                    const uint32_t sp = __builtin_amdgcn_perm(d, d, 0x0C000C00u | ((2u * j + 1u) << 16) | (2u * j));
-                    const f16x2 k1024 = {(f16)1024.f, (f16)1024.f};
-                    f16x2 qa = as_h2((sp & 0x000F000Fu) | 0x64006400u) - k1024;
-                    f16x2 qb = as_h2(((sp >> 4) & 0x000F000Fu) | 0x64006400u) - k1024;
-                    if constexpr (DQ) {  // one rounding each: fma in fp16
-                        qa = __builtin_elementwise_fma(qa, sc2, bi2);
-                        qb = __builtin_elementwise_fma(qb, sc2, bi2);
+                    const uint32_t dd[4] = {Wn[hb][j].x, Wn[hb][j].y, Wn[hb][j].z, Wn[hb][j].w};
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        f16x2 o[4];
+                        unpack_q8(dd[2 * h], dd[2 * h + 1], o);
+                        if constexpr (DQ) {  // 32-group 4 c + 2 j + h: the scale in half h of word 2 c + j
+                            const f16 sc = h ? as_h2(Dn[hb][j]).y : as_h2(Dn[hb][j]).x;
+                            const f16x2 sc2 = {sc, sc};
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) o[i] = o[i] * sc2;
+                        }
+                        Bs[b][sr][2 * j + h][lane] = pack4(o);
                     }
-                    o[j] = h2_bits(qa);
-                    o[2 + j] = h2_bits(qb);
                 }
-                Bs[b][sr][2 * gg + (slot >> 1)][r + 16 * (2 * (slot & 1) + h)] = make_uint4(o[0], o[1], o[2], o[3]);
+            } else {
+                // Dword 2 gg + h of a lane is k-step 2 gg + h.
+                const uint32_t dd[4] = {Wn[hb][0].x, Wn[hb][0].y, Wn[hb][0].z, Wn[hb][0].w};
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    f16x2 o[4];
+                    unpack_q4(dd[j], o);
+                    if constexpr (DQ) {  // 64-group 2 c + j / 2: (scale, bias); one rounding each, fma in fp16
+                        const f16x2 sbw = as_h2(Dn[hb][j >> 1]);
+                        const f16x2 sc2 = {sbw.x, sbw.x}, bi2 = {sbw.y, sbw.y};
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) o[i] = __builtin_elementwise_fma(o[i], sc2, bi2);
+                    }
+                    Bs[b][sr][j][lane] = pack4(o);
+                }
             }
         }
-        }
-      }
         if constexpr (!DQ) Vs[b][tid] = Vn;
     };
     // One activation operand (token block tb0 + i, k-step kk of group g, hi / lo part hl).
@@ -410,14 +515,9 @@ __global__ __launch_bounds__(512) void pf_gemm_kernel(PfGemmArgs a) {
             v8h Xh[TB], Xl[TB], Bb[4];
 #pragma unroll
             for (int i = 0; i < TB; ++i) {
-                const float* xp = a.xs + ((size_t)(tb0 + i) * NG + 32 * cg + 8 * q) * 16 + r16;
-#pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    const float x = xp[16 * j] * 0.00390625f;  // 2^-8: a group sum of 64 values below 2^15
-                    const f16 hx = (f16)x;
-                    Xh[i][j] = hx;
-                    Xl[i][j] = (f16)(x - (float)hx);
-                }
+                const uint16_t* xp = a.xb + ((size_t)((tb0 + i) * (NG / 32) + cg) * 2 * 64 + lane) * 8;
+                Xh[i] = *(const v8h*)xp;
+                Xl[i] = *(const v8h*)(xp + 512);
             }
 #pragma unroll
             for (int hf = 0; hf < NHF; ++hf) {
@@ -467,26 +567,297 @@ __global__ __launch_bounds__(512) void pf_gemm_kernel(PfGemmArgs a) {
             const int row = tn * TR + rb * 16 + r16;
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                const int t = tq + e;
-                const float y = acc[i][r][e] * tsc[e];
-                if constexpr (EPI == EPI_STORE) {
-                    if (t < a.M) a.y[(size_t)t * a.N + row] = y;
-                } else if constexpr (EPI == EPI_RESID) {
-                    if (t < a.M) {
-                        float* xo = a.y + (size_t)t * a.N + row;
-                        float v = *xo + y;
-                        if (a.ds) {  // DeepStack residual of a visual row (Shaders.swift:696-707)
-                            const int vrow = a.row0 + t - a.vis_offset;
-                            if (a.vis_offset >= 0 && vrow >= 0 && vrow < a.n_vis) v = v + a.ds[(size_t)vrow * H + row];
-                        }
-                        *xo = v;
-                    }
-                } else {  // EPI_SWIGLU: block RB tn + rb = gate units 8 (RB tn + rb) + 0..7, then their up rows
-                    const float up = dpp<0x128>(y);  // lane r16 ^ 8 of the row of 16 (a rotation by 8)
-                    const float hv = y * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-y * 1.4426950408889634f)) * up;
-                    if (t < a.M && r16 < 8) a.h[(size_t)t * FF + (tn * PG_RB + rb) * 8 + r16] = hv;
+                pf_store<EPI>(a, tq + e, row, acc[i][r][e] * tsc[e]);
+            }
+        }
+    }
+}
+
+// ------------------------------------------------------------------------------------------
+// GEMM of prompts whose 128-token tiles leave the chip idle: K split over workgroups.
+//
+// A workgroup of 8 waves computes 16 TB tokens x 64 WN weight rows over a range of K: wave w owns
+// row blocks 4 (w / WK) .. + 3 and every WK-th K unit of KU values (WK = 8 / WN), all tokens.  So
+// a wave's weights are its own: they go from HBM to its registers (one unit ahead) and become B
+// operands there, with no LDS round trip and no sharing.  The activation operands, which the WN
+// row groups share, go to LDS by direct global-to-LDS loads, one iteration (WK units) ahead, in
+// operand order (1 KiB per fragment, no bank conflicts).  One barrier an iteration.  At the end
+// the WK waves of a row group add their sums through LDS (a fixed order).
+//
+// With a.splits > 1 the workgroup stores its sums as partials [split][M][N] and the kernel that
+// consumes the result adds them (prep, q/k norm): no atomics, the same sums on every run.
+//
+// Workgroups run row tile by row tile on one XCD (token tiles innermost), so that the weights
+// cross HBM once.
+template <int FMT, int K, int EPI, int TB, int HL, int WN>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void pf_split_kernel(PfGemmArgs a) {
+    constexpr int WK = 8 / WN, NG = K / 64, NKS = K / 32, NXB = (NG + 31) / 32;
+    // k-steps of a unit (KU = 32 KSU): a q4 chunk's 128 K, or 64 where that would not leave LDS for two stages.
+    constexpr int KSU = FMT == FMT_Q4 && WN == 4 ? 4 : 2;
+    constexpr int CPU = FMT == FMT_F16 ? 2 : 1;                     // 1 KiB weight chunks of a unit
+    constexpr bool HALFCH = FMT == FMT_Q4 && KSU == 2;              // a unit is half a chunk (8 bytes a lane)
+    constexpr int IKS = WK * KSU, NIT = NKS / IKS;                  // k-steps of an iteration, iterations of K
+    constexpr int ACH = IKS * HL * TB, AW = ACH / 8;                // 1 KiB operand chunks of a stage, per wave
+    constexpr int UN = TB * 4, UW = UN / WK;                        // 16 x 16 blocks of a wave's tile, finished per wave
+    constexpr int REDCH = WN * UN * (WK - 1);                       // KiB of the final exchange
+    constexpr int LDSB = (2 * ACH > REDCH ? 2 * ACH : REDCH) * 1024;
+    constexpr bool DQ = HL == 1 || FMT == FMT_F16;
+    static_assert(NKS % IKS == 0 && ACH % 8 == 0 && UN % WK == 0 && (UW == 2 || UW % 4 == 0) && LDSB <= 160 * 1024, "shape");
+    __shared__ __align__(1024) uint8_t lds[LDSB];
+
+    const int TN = a.N / (64 * WN), TM = (a.M + 16 * TB - 1) / (16 * TB), T = TM * TN * a.splits;
+    const int per = (T + 7) / 8;
+    const int tile = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);
+    if (tile >= T) return;
+    const int tm = tile % TM, sk = (tile / TM) % a.splits, tn = tile / TM / a.splits;
+    const int it0 = sk * NIT / a.splits, it1 = (sk + 1) * NIT / a.splits;
+
+    // The wave's index in a scalar register: its base addresses are scalar, its lanes add 32-bit offsets.
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), q = lane >> 4, r16 = lane & 15;
+    const int wn = wave / WK, part = wave % WK;
+    const int tb0 = tm * TB, rb0 = (tn * WN + wn) * 4;
+
+    // A stage: chunk ((ks HL) + hl) TB + tb of the iteration's k-steps.
+    // Buffer resources: a request is a scalar offset plus the lane's (no 64-bit lane addresses).
+    const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)(a.xa + (size_t)tb0 * NKS * HL * 512), (short)0, TB * NKS * HL * 1024, 0x00020000);
+    auto aload = [&](int st, int it) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < AW; ++u) {
+            const int ch = wave + 8 * u, tb = ch % TB, kh = ch / TB;  // kh = ks HL + hl
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(xrs, (__attribute__((address_space(3))) void*)(lds + (st * ACH + ch) * 1024),
+                                                     16, lane * 16, (tb * NKS * HL + it * IKS * HL + kh) * 1024, 0, 0);
+        }
+    };
+    // Weights of one unit: row blocks rb0 .. + 3, and their scale words (q4 (scale, bias) of the
+    // unit's two 64-groups; q8 the scales of its two 32-groups).
+    struct Unit {
+        uint4 w[4][CPU];
+        uint2 s[4];
+    };
+    constexpr int RBW = FMT == FMT_Q4 ? K * 8 : FMT == FMT_Q8 ? K * 16 : K * 32;  // bytes of a row block's codes
+    const uint8_t* sp = a.sb + (size_t)rb0 * 16 * NG * 4;  // (unused for f16)
+    const __amdgpu_buffer_rsrc_t wrs =
+        __builtin_amdgcn_make_buffer_rsrc((void*)(a.w + (size_t)rb0 * RBW), (short)0, 4 * RBW, 0x00020000);
+    const __amdgpu_buffer_rsrc_t srs = __builtin_amdgcn_make_buffer_rsrc((void*)sp, (short)0, 64 * NG * 4, 0x00020000);
+    const int wlane = lane * 16, slane = r16 * NG * 4;
+    auto wload = [&](int it, Unit& u) __attribute__((always_inline)) {
+        const int un = it * WK + part;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            if constexpr (HALFCH) {
+                const uint2 h = __builtin_bit_cast(
+                    uint2, __builtin_amdgcn_raw_buffer_load_b64(wrs, wlane, r * RBW + (un >> 1) * 1024 + (un & 1) * 8, 0));
+                u.w[r][0].x = h.x;
+                u.w[r][0].y = h.y;
+                u.s[r].x = __builtin_amdgcn_raw_buffer_load_b32(srs, slane, r * 16 * NG * 4 + un * 4, 0);
+                continue;
+            }
+#pragma unroll
+            for (int c = 0; c < CPU; ++c)
+                u.w[r][c] = __builtin_bit_cast(
+                    uint4, __builtin_amdgcn_raw_buffer_load_b128(wrs, wlane, r * RBW + (un * CPU + c) * 1024, 0));
+            if constexpr (FMT == FMT_Q4)
+                u.s[r] = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(srs, slane, r * 16 * NG * 4 + un * 8, 0));
+            if constexpr (FMT == FMT_Q8)
+                u.s[r].x = __builtin_amdgcn_raw_buffer_load_b32(srs, slane, r * 16 * NG * 4 + un * 4, 0);
+        }
+    };
+
+    f32x4 acc[TB][4];
+#pragma unroll
+    for (int i = 0; i < TB; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[i][r] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+    Unit un;
+    aload(0, it0);
+    wload(it0, un);
+    if constexpr (FMT == FMT_Q4 && !DQ) {
+        // The q4 bias term sum_g b_g X_g over the range's groups, on the matrix cores: 32 groups are
+        // one k-step, A = the group sums (times 2^-8, hi + lo), B = the rows' fp16 biases, exact.  The
+        // sums stay 2^-8 of their value until the end (the loop's scales are taken down with them).
+        // Biases outside the range are requested past the buffer's end, which gives zeros (ranges
+        // are whole fours of groups).
+        const int g0 = it0 * IKS / 2, g1 = it1 * IKS / 2;
+#pragma unroll 1
+        for (int cg = g0 / 32; cg < (g1 + 31) / 32; ++cg) {
+            if (cg % WK != part) continue;
+            v8h Xh[TB], Xl[TB];
+            uint4 w0[4], w1[4];
+#pragma unroll
+            for (int i = 0; i < TB; ++i) {
+                const uint16_t* xp = a.xb + (size_t)((tb0 + i) * NXB + cg) * 2 * 64 * 8;
+                Xh[i] = *(const v8h*)(xp + lane * 8);
+                Xl[i] = *(const v8h*)(xp + 512 + lane * 8);
+            }
+            const int g = 32 * cg + 8 * q;
+            const int o0 = g >= g0 && g < g1 ? slane + g * 4 : (int)0x80000000, o1 = g + 4 >= g0 && g + 4 < g1 ? slane + g * 4 + 16 : (int)0x80000000;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                w0[r] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(srs, o0 + r * 16 * NG * 4, 0, 0));
+                w1[r] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(srs, o1 + r * 16 * NG * 4, 0, 0));
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const uint4 b = make_uint4(__builtin_amdgcn_perm(w0[r].y, w0[r].x, 0x07060302u), __builtin_amdgcn_perm(w0[r].w, w0[r].z, 0x07060302u),
+                                           __builtin_amdgcn_perm(w1[r].y, w1[r].x, 0x07060302u), __builtin_amdgcn_perm(w1[r].w, w1[r].z, 0x07060302u));
+#pragma unroll
+                for (int i = 0; i < TB; ++i) {
+                    acc[i][r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Xh[i], __builtin_bit_cast(v8h, b), acc[i][r], 0, 0, 0);
+                    acc[i][r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Xl[i], __builtin_bit_cast(v8h, b), acc[i][r], 0, 0, 0);
                 }
             }
+        }
+    }
+
+    // One unit against the operands of stage st.
+    auto mac = [&](int st, Unit u) __attribute__((always_inline)) {
+        const uint8_t* A0 = lds + (size_t)(st * ACH + part * KSU * HL * TB) * 1024 + lane * 16;
+#pragma unroll 1
+        for (int g = 0; g < KSU / 2; ++g, A0 += 2 * HL * TB * 1024) {  // 64 K
+            v8h A[2][HL][TB];
+#pragma unroll
+            for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+                for (int hl = 0; hl < HL; ++hl)
+#pragma unroll
+                    for (int i = 0; i < TB; ++i)
+                        A[kk][hl][i] = *(const v8h*)(A0 + (size_t)((kk * HL + hl) * TB + i) * 1024);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                v8h B[2];
+                float s0 = 1.f, s1 = 1.f;
+                if constexpr (FMT == FMT_F16) {
+#pragma unroll
+                    for (int kk = 0; kk < 2; ++kk) B[kk] = __builtin_bit_cast(v8h, u.w[r][kk]);
+                } else {
+                    const uint32_t dd[4] = {u.w[r][0].x, u.w[r][0].y, u.w[r][0].z, u.w[r][0].w};
+                    const f16x2 sw = as_h2(u.s[r].x);
+#pragma unroll
+                    for (int kk = 0; kk < 2; ++kk) {
+                        f16x2 o[4];
+                        if constexpr (FMT == FMT_Q4)
+                            unpack_q4(dd[kk], o);
+                        else
+                            unpack_q8(dd[2 * kk], dd[2 * kk + 1], o);
+                        if constexpr (DQ) {  // one rounding each, as the 128-token tiles
+                            const f16x2 sc2 = FMT == FMT_Q8 && kk ? f16x2{sw.y, sw.y} : f16x2{sw.x, sw.x};
+                            const f16x2 bi2 = {sw.y, sw.y};
+#pragma unroll
+                            for (int i = 0; i < 4; ++i)
+                                o[i] = FMT == FMT_Q4 ? __builtin_elementwise_fma(o[i], sc2, bi2) : o[i] * sc2;
+                        }
+                        B[kk] = __builtin_bit_cast(v8h, pack4(o));
+                    }
+                    s0 = FMT == FMT_Q4 ? (float)sw.x * 0.00390625f : (float)sw.x;
+                    s1 = (float)sw.y;
+                }
+                if constexpr (DQ) {
+#pragma unroll
+                    for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+                        for (int hl = 0; hl < HL; ++hl)
+#pragma unroll
+                            for (int i = 0; i < TB; ++i)
+                                acc[i][r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[kk][hl][i], B[kk], acc[i][r], 0, 0, 0);
+                } else {
+                    f32x4 C[TB];
+#pragma unroll
+                    for (int kk = 0; kk < 2; ++kk) {
+                        if (FMT == FMT_Q8 || kk == 0) {
+#pragma unroll
+                            for (int i = 0; i < TB; ++i) C[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+                        }
+#pragma unroll
+                        for (int hl = 0; hl < HL; ++hl)
+#pragma unroll
+                            for (int i = 0; i < TB; ++i)
+                                C[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[kk][hl][i], B[kk], C[i], 0, 0, 0);
+                        if (FMT == FMT_Q8 || kk == 1) {
+                            const float s = FMT == FMT_Q8 && kk ? s1 : s0;
+#pragma unroll
+                            for (int i = 0; i < TB; ++i)
+#pragma unroll
+                                for (int e = 0; e < 4; ++e) acc[i][r][e] = fmaf(s, C[i][e], acc[i][r][e]);
+                        }
+                    }
+                }
+                if constexpr (FMT == FMT_Q4) {  // the unit's second 64-group moves down
+                    u.w[r][0].x = u.w[r][0].z;
+                    u.w[r][0].y = u.w[r][0].w;
+                    u.s[r].x = u.s[r].y;
+                }
+            }
+        }
+    };
+    // Every load of the iteration was issued an iteration ago: wait for this wave's, then for every
+    // wave's; the barrier also frees the stage read in the iteration before.
+    auto arrive = [&]() __attribute__((always_inline)) {
+        __builtin_amdgcn_s_waitcnt(0);
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    for (int it = it0; it < it1; ++it) {
+        arrive();
+        const Unit u = un;  // landed: the copy waits for nothing, and its registers take the next unit
+        const int st = (it - it0) & 1;
+        if (it + 1 < it1) {
+            aload(st ^ 1, it + 1);
+            wload(it + 1, un);
+        }
+        mac(st, u);
+    }
+
+    // The row group's WK sums: block u (token block u / 4, row block u % 4) is finished by part u / UW.
+    // (The code of a launch that lasts microseconds is fetched once per CU, so its length counts.)
+    f32x4 sum[UW];
+    {
+        f32x4* red = (f32x4*)lds + (size_t)wn * UN * (WK - 1) * 64 + lane;
+        __syncthreads();  // every operand read is done (no load is in flight)
+#pragma unroll
+        for (int p = 0; p < WK; ++p) {
+#pragma unroll
+            for (int i = 0; i < UW; ++i) {
+                const int u = p * UW + i;
+                if (p == part)
+                    sum[i] = acc[u / 4][u % 4];
+                else
+                    red[(size_t)(u * (WK - 1) + (part < p ? part : part - 1)) * 64] = acc[u / 4][u % 4];
+            }
+        }
+        __syncthreads();
+        red += (size_t)part * UW * (WK - 1) * 64;
+#pragma unroll
+        for (int i = 0; i < UW; ++i)
+#pragma unroll
+            for (int p = 0; p < WK - 1; ++p) {
+                const f32x4 o = red[(i * (WK - 1) + p) * 64];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) sum[i][e] += o[e];
+            }
+    }
+    // Lane: tokens 16 tb + 4 q + e of weight row 16 rb + r16.  Rows of tokens past M are past the
+    // end of the destination's buffer resource and are dropped (the whole offset is the lane's: a
+    // scalar offset past the end would wrap the bounds check).
+    constexpr float UNBIAS = FMT == FMT_Q4 && !DQ ? 256.f : 1.f;
+    const int tb1 = tb0 + part * UW / 4, r1 = part * UW % 4;  // UW is 2 or a multiple of 4
+    float* dst = a.splits > 1 ? a.part + (size_t)sk * a.M * a.N : a.y;
+    const __amdgpu_buffer_rsrc_t drs =
+        __builtin_amdgcn_make_buffer_rsrc((void*)dst, (short)0, (int)((size_t)a.M * a.N * 4), 0x00020000);
+#pragma unroll
+    for (int i = 0; i < UW; ++i) {
+        const int tq = (tb1 + i / 4) * 16, rb = rb0 + (UW < 4 ? r1 + i : i % 4);
+        const float4 tsv = *(const float4*)(a.ts + tq + 4 * q);
+        const float tsc[4] = {tsv.x, tsv.y, tsv.z, tsv.w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float y = sum[i][e] * (tsc[e] * UNBIAS);
+            if (EPI == EPI_STORE || a.splits > 1)
+                __builtin_amdgcn_raw_buffer_store_b32(as_u32(y), drs, ((tq + 4 * q + e) * a.N + rb * 16 + r16) * 4, 0, 0);
+            else
+                pf_store<EPI>(a, tq + 4 * q + e, rb * 16 + r16, y);
         }
     }
 }
@@ -500,10 +871,17 @@ __global__ __launch_bounds__(256) void pf_qk_kernel(PfQkArgs a) {
     const int t = blockIdx.x, lane = threadIdx.x % 64, vec = blockIdx.y * 4 + threadIdx.x / 64;
     if (t >= a.M) return;
     const int slot = a.p0 + t;
-    const float* row = a.qkv + (size_t)t * QKV;
+    // The vector's two elements of this lane (vectors are q heads, k groups, v groups in row order),
+    // the sum of the QKV GEMM's K-split partials.
+    const float* row = a.qkv + (size_t)t * QKV + vec * HD + lane;
+    float x0 = row[0], x1 = row[64];
+#pragma unroll 4
+    for (int s = 1; s < a.nsplit; ++s) {
+        x0 += row[(size_t)s * a.M * QKV];
+        x1 += row[(size_t)s * a.M * QKV + 64];
+    }
     const float* cs = a.rope + (size_t)slot * 128;
     if (vec < NH) {
-        float x0 = row[vec * HD + lane], x1 = row[vec * HD + lane + 64];
         norm_rope_pair(x0, x1, a.q_norm, cs, lane);
         // 1/sqrt(128) and log2(e): the scores come out in base-2 units, so every softmax
         // exponential of the attention is one v_exp_f32.
@@ -520,17 +898,15 @@ __global__ __launch_bounds__(256) void pf_qk_kernel(PfQkArgs a) {
         }
     } else if (vec < NH + NKV) {
         const int g = vec - NH;
-        float k0 = row[H + g * HD + lane], k1 = row[H + g * HD + lane + 64];
-        norm_rope_pair(k0, k1, a.k_norm, cs, lane);
+        norm_rope_pair(x0, x1, a.k_norm, cs, lane);
         uint16_t* kd = a.kc + ((size_t)g * a.maxctx + slot) * HD;
-        kd[lane] = f2h(k0);
-        kd[lane + 64] = f2h(k1);
+        kd[lane] = f2h(x0);
+        kd[lane + 64] = f2h(x1);
     } else {
         const int g = vec - NH - NKV;
-        const float* v = row + H + NKV * HD + g * HD;
         uint16_t* vd = a.vc + ((size_t)g * a.maxctx + slot) * HD;
-        vd[lane] = f2h(v[lane]);
-        vd[lane + 64] = f2h(v[lane + 64]);
+        vd[lane] = f2h(x0);
+        vd[lane + 64] = f2h(x1);
     }
 }
 
@@ -543,6 +919,10 @@ __global__ __launch_bounds__(256) void pf_qk_kernel(PfQkArgs a) {
 // running softmax states, merged through LDS after the last iteration.  Slots at or beyond the
 // block's last query are masked for all of its queries; causal masking uses cache slots.  The
 // softmax denominators come from the matrix cores too: a ones operand against the probabilities.
+//
+// With a.nsplit > 1 (few query blocks) a block's key iterations are dealt to nsplit workgroups,
+// each storing its unnormalised rows and their (maximum, denominator); the operand prep of the O
+// projection merges them.
 
 typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
@@ -557,7 +937,7 @@ template <int HL>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void pf_attn_kernel(PfAttnArgs a) {
     extern __shared__ __align__(16) uint16_t pa_lds[];
     const int QB = (a.M + 63) / 64;
-    const int g = (int)(blockIdx.x % NKV), qb = QB - 1 - (int)(blockIdx.x / NKV);
+    const int g = (int)(blockIdx.x % NKV), qs = (int)(blockIdx.x / NKV), qb = QB - 1 - qs / a.nsplit, sp = qs % a.nsplit;
     if (qb < 0) return;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, q = lane >> 4, r16 = lane & 15;
     const int par = wave >> 2, wi = wave & 3;
@@ -566,6 +946,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const int kv_lim = a.p0 + min(a.M, qb * 64 + 64);  // past the block's last query slot
     const int nkb = (kv_lim - 1) / PA_KB + 1;          // 64-slot key halves with unmasked keys
     const int nit = (nkb + 1) / 2;
+    const int it0 = sp * nit / a.nsplit, it1 = (sp + 1) * nit / a.nsplit;  // may be empty
     const bool active = t0 < a.M;
     const int w_first = a.p0 + t0;
     const int w_last = a.p0 + min(a.M - 1, t0 + 31);
@@ -644,12 +1025,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const f16 one = (f16)1.0f;
     const v8h ones = {one, one, one, one, one, one, one, one};
 
-    gload(0);
+    gload(it0);
     lstore(0);
     __syncthreads();
-    for (int it = 0; it < nit; ++it) {
-        const int st = it & 1;
-        if (it + 1 < nit) gload(it + 1);
+    for (int it = it0; it < it1; ++it) {
+        const int st = (it - it0) & 1;
+        if (it + 1 < it1) gload(it + 1);
         const int kb = 2 * it + par;
         if (active && kb * PA_KB <= w_last) {
             const uint16_t* Ks = pa_lds + (2 * st + par) * PA_BUF;
@@ -772,12 +1153,13 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                 }
             }
         }
-        if (it + 1 < nit) lstore(st ^ 1);
+        if (it + 1 < it1) lstore(st ^ 1);
         __syncthreads();
     }
 
     // Key-parity merge: waves 4..7 hand (O, m, l) to waves 0..3 through LDS (free after the loop's
-    // last barrier).  Waves 0..3 always have a finite maximum: half 0 holds key slot 0.
+    // last barrier).  Unsplit, waves 0..3 always have a finite maximum: half 0 holds key slot 0.  A
+    // split may see no key of a query: its maximum stays -inf, its sums 0.
     float* mo = (float*)pa_lds;               // [4 waves][2 tiles][8 dim tiles][64 lanes] x 4
     float* mml = mo + 4 * 2 * 8 * 64 * 4;     // [4 waves][2 tiles][64 lanes] x (m, l)
     if (par == 1) {
@@ -797,14 +1179,17 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             const float m = fmaxf(m_run[u], ml1.x);
             const float f0 = m == m_run[u] ? 1.f : __builtin_amdgcn_exp2f(m_run[u] - m);
             const float f1 = ml1.x == -__builtin_inff() ? 0.f : __builtin_amdgcn_exp2f(ml1.x - m);
-            const float inv = 1.0f / (Lr[u][0] * f0 + ml1.y * f1);
+            const float l = Lr[u][0] * f0 + ml1.y * f1;
+            const float inv = a.nsplit > 1 ? 1.0f : 1.0f / l;
+            float* out = a.nsplit > 1 ? a.part + (size_t)sp * a.M * H : a.out;
             if (t < a.M) {
+                if (a.nsplit > 1 && q == 0) ((float2*)a.part_ml)[((size_t)sp * a.M + t) * NH + head] = make_float2(m, l);
 #pragma unroll
                 for (int dt = 0; dt < 8; ++dt) {
                     const f32x4 o1 = *(const f32x4*)(mo + (((wi * 2 + u) * 8 + dt) * 64 + lane) * 4);
                     const float4 o = make_float4((O[u][dt][0] * f0 + o1[0] * f1) * inv, (O[u][dt][1] * f0 + o1[1] * f1) * inv,
                                                  (O[u][dt][2] * f0 + o1[2] * f1) * inv, (O[u][dt][3] * f0 + o1[3] * f1) * inv);
-                    *(float4*)(a.out + (size_t)t * H + head * HD + dt * 16 + 4 * q) = o;
+                    *(float4*)(out + (size_t)t * H + head * HD + dt * 16 + 4 * q) = o;
                 }
             }
         }
@@ -813,25 +1198,36 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 
 // ------------------------------------------------------------------------------------------
 
-template <int HL>
-static hipError_t pf_prep_hl(int K, int norm, const float* src, const float* norm_w, int M, int Mpad, uint16_t* xa,
-                             float* xs, float* ts, hipStream_t s) {
-    if (K == H && norm)
-        hipLaunchKernelGGL((pf_prep_kernel<H, true, HL>), dim3(Mpad), dim3(256), 0, s, src, norm_w, M, xa, xs, ts);
-    else if (K == H)
-        hipLaunchKernelGGL((pf_prep_kernel<H, false, HL>), dim3(Mpad), dim3(256), 0, s, src, norm_w, M, xa, xs, ts);
-    else if (K == FF && !norm)
-        hipLaunchKernelGGL((pf_prep_kernel<FF, false, HL>), dim3(Mpad), dim3(256), 0, s, src, norm_w, M, xa, xs, ts);
+template <int K, int SRC>
+static hipError_t pf_prep_src(int fmt, const PfPrepArgs& a, hipStream_t s) {
+    const dim3 grid(a.Mpad), block(256);
+    if (a.parts == 2 && fmt == FMT_Q4)
+        hipLaunchKernelGGL((pf_prep_kernel<K, SRC, 2, true>), grid, block, 0, s, a);
+    else if (a.parts == 2)
+        hipLaunchKernelGGL((pf_prep_kernel<K, SRC, 2, false>), grid, block, 0, s, a);
+    else if (fmt == FMT_Q4)
+        hipLaunchKernelGGL((pf_prep_kernel<K, SRC, 1, true>), grid, block, 0, s, a);
     else
-        return hipErrorInvalidValue;
+        hipLaunchKernelGGL((pf_prep_kernel<K, SRC, 1, false>), grid, block, 0, s, a);
     return hipGetLastError();
 }
 
-hipError_t launch_pf_prep(int K, int norm, const float* src, const float* norm_w, int M, int Mpad, uint16_t* xa,
-                          float* xs, float* ts, int parts, hipStream_t s) {
-    if (M < 1 || Mpad < M || Mpad % 128 || (parts != 1 && parts != 2)) return hipErrorInvalidValue;
-    return parts == 2 ? pf_prep_hl<2>(K, norm, src, norm_w, M, Mpad, xa, xs, ts, s)
-                      : pf_prep_hl<1>(K, norm, src, norm_w, M, Mpad, xa, xs, ts, s);
+hipError_t launch_pf_prep(int fmt, int src, const PfPrepArgs& a, hipStream_t s) {
+    if (a.M < 1 || a.Mpad < a.M || a.Mpad % 8 || (a.parts != 1 && a.parts != 2) || a.nsplit < 0 ||
+        (a.nsplit > 0 && !a.part))
+        return hipErrorInvalidValue;
+    switch (src) {
+        case PF_SRC_RESID: return pf_prep_src<H, PF_SRC_RESID>(fmt, a, s);
+        case PF_SRC_ATTN: return pf_prep_src<H, PF_SRC_ATTN>(fmt, a, s);
+        case PF_SRC_SWIGLU: return pf_prep_src<FF, PF_SRC_SWIGLU>(fmt, a, s);
+    }
+    return hipErrorInvalidValue;
+}
+
+hipError_t launch_pf_last_row(const PfPrepArgs& a, int t, hipStream_t s) {
+    if (t < 0 || t >= a.M || a.nsplit < 0) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(pf_last_row_kernel, dim3(H / 256), dim3(256), 0, s, a, t);
+    return hipGetLastError();
 }
 
 template <int FMT, int RB, int TB, int HL>
@@ -874,9 +1270,68 @@ static hipError_t pf_gemm_fmt(int K, int epi, const PfGemmArgs& a, hipStream_t s
     return pf_gemm_shape<FMT, 8, 1>(K, epi, a, s);
 }
 
-hipError_t launch_pf_gemm(int fmt, int K, int epi, const PfGemmArgs& a, hipStream_t s) {
-    if (a.M < 1 || a.Mpad < a.M || a.Mpad % 128 || a.N % 128 || (a.parts != 1 && a.parts != 2))
+template <int FMT, int TB, int HL, int WN>
+static hipError_t pf_split_shape(int K, int epi, const PfGemmArgs& a, hipStream_t s) {
+    const int T = ((a.M + 16 * TB - 1) / (16 * TB)) * (a.N / (64 * WN)) * a.splits;
+    const dim3 grid(8 * ((T + 7) / 8)), block(512);
+    if (K == H && epi == EPI_STORE)
+        hipLaunchKernelGGL((pf_split_kernel<FMT, H, EPI_STORE, TB, HL, WN>), grid, block, 0, s, a);
+    else if (K == H && epi == EPI_RESID)
+        hipLaunchKernelGGL((pf_split_kernel<FMT, H, EPI_RESID, TB, HL, WN>), grid, block, 0, s, a);
+    else if (K == H && epi == EPI_SWIGLU)
+        hipLaunchKernelGGL((pf_split_kernel<FMT, H, EPI_SWIGLU, TB, HL, WN>), grid, block, 0, s, a);
+    else if (K == FF && epi == EPI_RESID)
+        hipLaunchKernelGGL((pf_split_kernel<FMT, FF, EPI_RESID, TB, HL, WN>), grid, block, 0, s, a);
+    else
         return hipErrorInvalidValue;
+    return hipGetLastError();
+}
+
+// Tiles of the K-split GEMM: 32 tokens (two token blocks) up to 32 rows, else 64; 128 weight rows
+// while there is one token tile, else 256 (a tile's operands are then shared by four row groups).
+struct PfSplitShape {
+    int tb, wn, nit;  // token blocks, row groups, iterations of K
+};
+static PfSplitShape pf_split_tile(int fmt, int K, int M) {
+    const int tb = M <= 32 ? 2 : 4, wn = M <= 64 ? 2 : 4;
+    const int unit = fmt == FMT_Q4 && wn == 4 ? 128 : 64;
+    return {tb, wn, K / (8 / wn * unit)};
+}
+
+template <int FMT>
+static hipError_t pf_split_fmt(int K, int epi, const PfGemmArgs& a, hipStream_t s) {
+    const PfSplitShape t = pf_split_tile(FMT, K, a.M);
+    if (a.parts == 1)
+        return t.tb == 2   ? pf_split_shape<FMT, 2, 1, 2>(K, epi, a, s)
+               : t.wn == 2 ? pf_split_shape<FMT, 4, 1, 2>(K, epi, a, s)
+                           : pf_split_shape<FMT, 4, 1, 4>(K, epi, a, s);
+    return t.tb == 2   ? pf_split_shape<FMT, 2, 2, 2>(K, epi, a, s)
+           : t.wn == 2 ? pf_split_shape<FMT, 4, 2, 2>(K, epi, a, s)
+                       : pf_split_shape<FMT, 4, 2, 4>(K, epi, a, s);
+}
+
+int pf_gemm_splits(int fmt, int K, int N, int M) {
+    if (!pf_use_split(M)) return 1;
+    const PfSplitShape t = pf_split_tile(fmt, K, M);
+    const int tiles = ((M + 16 * t.tb - 1) / (16 * t.tb)) * (N / (64 * t.wn));
+    const int most = std::max(1, std::min(t.nit, 256 / tiles));
+    const int its = (t.nit + most - 1) / most;
+    return (t.nit + its - 1) / its;
+}
+
+hipError_t launch_pf_gemm(int fmt, int K, int epi, const PfGemmArgs& a, hipStream_t s) {
+    if (a.M < 1 || a.N % 256 || (a.parts != 1 && a.parts != 2) || a.splits < 1 || (a.splits > 1 && !a.part))
+        return hipErrorInvalidValue;
+    if (pf_use_split(a.M)) {
+        if (a.splits != pf_gemm_splits(fmt, K, a.N, a.M) || a.Mpad < (a.M + 63) / 64 * 64) return hipErrorInvalidValue;
+        switch (fmt) {
+            case FMT_Q4: return pf_split_fmt<FMT_Q4>(K, epi, a, s);
+            case FMT_Q8: return pf_split_fmt<FMT_Q8>(K, epi, a, s);
+            case FMT_F16: return pf_split_fmt<FMT_F16>(K, epi, a, s);
+        }
+        return hipErrorInvalidValue;
+    }
+    if (a.Mpad < a.M || a.Mpad % 128 || a.splits != 1) return hipErrorInvalidValue;
     switch (fmt) {
         case FMT_Q4: return pf_gemm_fmt<FMT_Q4>(K, epi, a, s);
         case FMT_Q8: return pf_gemm_fmt<FMT_Q8>(K, epi, a, s);
@@ -886,13 +1341,19 @@ hipError_t launch_pf_gemm(int fmt, int K, int epi, const PfGemmArgs& a, hipStrea
 }
 
 hipError_t launch_pf_qk(const PfQkArgs& a, hipStream_t s) {
-    if (a.M < 1 || a.p0 < 0 || a.p0 + a.M > a.maxctx) return hipErrorInvalidValue;
+    if (a.M < 1 || a.p0 < 0 || a.p0 + a.M > a.maxctx || a.nsplit < 1) return hipErrorInvalidValue;
     hipLaunchKernelGGL(pf_qk_kernel, dim3(a.M, (NH + 2 * NKV) / 4), dim3(256), 0, s, a);
     return hipGetLastError();
 }
 
+int pf_attn_splits(int M, int p0) {
+    const int QB = (M + 63) / 64, nit = (p0 + M + 2 * PA_KB - 1) / (2 * PA_KB);  // iterations of the last block
+    return std::max(1, std::min(nit, 256 / (QB * NKV)));
+}
+
 hipError_t launch_pf_attn(const PfAttnArgs& a, hipStream_t s) {
-    if (a.M < 1 || a.p0 < 0 || a.p0 + a.M > a.maxctx) return hipErrorInvalidValue;
+    if (a.M < 1 || a.p0 < 0 || a.p0 + a.M > a.maxctx || a.nsplit < 1 || (a.nsplit > 1 && (!a.part || !a.part_ml)))
+        return hipErrorInvalidValue;
     static bool attr_set = false;
     if (!attr_set) {
         for (const void* k : {(const void*)pf_attn_kernel<1>, (const void*)pf_attn_kernel<2>}) {
@@ -901,11 +1362,11 @@ hipError_t launch_pf_attn(const PfAttnArgs& a, hipStream_t s) {
         }
         attr_set = true;
     }
-    const int QB = (a.M + 63) / 64;
+    const dim3 grid((a.M + 63) / 64 * NKV * a.nsplit);
     if (a.ql)
-        hipLaunchKernelGGL(pf_attn_kernel<2>, dim3(QB * NKV), dim3(512), PA_LDS, s, a);
+        hipLaunchKernelGGL(pf_attn_kernel<2>, grid, dim3(512), PA_LDS, s, a);
     else
-        hipLaunchKernelGGL(pf_attn_kernel<1>, dim3(QB * NKV), dim3(512), PA_LDS, s, a);
+        hipLaunchKernelGGL(pf_attn_kernel<1>, grid, dim3(512), PA_LDS, s, a);
     return hipGetLastError();
 }
 

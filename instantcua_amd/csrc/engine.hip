@@ -809,7 +809,7 @@ struct icua_engine {
         g.sb = w.wqkv_sb;
         g.N = QKV;
         g.y = pqkv;
-        g.splits = pf_gemm_splits(fmt, H, QKV, M);
+        g.splits = pf_gemm_splits(fmt, parts, H, QKV, M);
         HIPCK(launch_pf_gemm(fmt, H, EPI_STORE, g, stream));
         // 2. q/k norm + M-RoPE + KV write, causal flash attention.
         uint16_t* ql = parts == 2 ? pql : nullptr;
@@ -827,7 +827,7 @@ struct icua_engine {
         g.sb = w.wo_sb;
         g.N = H;
         g.y = px;
-        g.splits = pf_gemm_splits(fmt, H, H, M);
+        g.splits = pf_gemm_splits(fmt, parts, H, H, M);
         HIPCK(launch_pf_gemm(fmt, H, EPI_RESID, g, stream));
         // 4. RMSNorm + gate|up + SwiGLU.
         p.src = px;
@@ -838,7 +838,7 @@ struct icua_engine {
         g.sb = w.wgu_sb;
         g.N = GU;
         g.h = ph;
-        g.splits = pf_gemm_splits(fmt, H, GU, M);
+        g.splits = pf_gemm_splits(fmt, parts, H, GU, M);
         HIPCK(launch_pf_gemm(fmt, H, EPI_SWIGLU, g, stream));
         // 5. Down projection + residual (+ DeepStack after layers 0-2 at visual rows).
         p.src = ph;
@@ -849,7 +849,7 @@ struct icua_engine {
         g.N = H;
         g.y = px;
         g.ds = (has_ds && l < 3) ? ds[l] : nullptr;
-        g.splits = pf_gemm_splits(fmt, FF, H, M);
+        g.splits = pf_gemm_splits(fmt, parts, FF, H, M);
         HIPCK(launch_pf_gemm(fmt, FF, EPI_RESID, g, stream));
         pend = g.splits > 1 ? PfPending{g.splits, g.ds} : PfPending{};
         return 0;
@@ -878,7 +878,8 @@ struct icua_engine {
         int M = 0;
         for (int c0 = 0; c0 < n; c0 += PF_CHUNK) {
             M = std::min(PF_CHUNK, n - c0);
-            const int pad = pf_use_split(M) ? 64 : 128, Mpad = (M + pad - 1) / pad * pad;
+            const int parts = (flags & ICUA_FLAG_PREFILL_FP16) ? 1 : 2;
+            const int pad = pf_use_split(fmt, parts, M) ? 64 : 128, Mpad = (M + pad - 1) / pad * pad;
             EmbedArgs ea{};
             ea.toks = prompt;
             ea.E = E;

@@ -145,10 +145,18 @@ struct PfGemmArgs {
     int splits;             // pf_gemm_splits(): > 1 stores K-split partials [splits][M][N] to part
     float* part;
 };
-// Prompts of up to PF_SPLIT_M rows take the K-split GEMM.
-constexpr int PF_SPLIT_M = 1024;
-inline bool pf_use_split(int M) { return M <= PF_SPLIT_M; }
-int pf_gemm_splits(int fmt, int K, int N, int M);
+// Chunks of up to this many rows take the K-split GEMM, larger ones the 128-token tiles, by the
+// weights and the operand parts.  The lines lie where the two meet (4 layers and the head, split /
+// 128-token tiles, ms): hi + lo q4 1.30 / 1.31 at 1000 rows, 2.12 / 2.27 at 1536, 2.55 / 2.37 at 2048
+// (q8 2.33 / 2.47 and 2.82 / 2.56); f16 2.71 / 2.77 at 2048 and 5.04 / 5.28 at 4096, ahead at every
+// size (its 128-token tiles are 128 rows wide).  fp16 operands alone: q4 1.30 / 1.36 at 1280,
+// 1.47 / 1.41 at 1536 (f16 1.62 / 1.70, 1.74 / 1.61); q8 0.85 / 0.87 at 512, 1.13 / 1.01 at 768.
+inline int pf_split_rows(int fmt, int parts) {
+    if (parts == 2) return fmt == FMT_F16 ? 4096 : 1536;
+    return fmt == FMT_Q8 ? 512 : 1280;
+}
+inline bool pf_use_split(int fmt, int parts, int M) { return M <= pf_split_rows(fmt, parts); }
+int pf_gemm_splits(int fmt, int parts, int K, int N, int M);
 // Partials of a GEMM (at most 256 tiles of 64 x 256) or an attention (256 / 8 query
 // blocks and splits of 64 rows), floats.
 constexpr size_t PF_PART_FLOATS = (size_t)256 * 64 * 256;

@@ -589,6 +589,12 @@ __global__ __launch_bounds__(512) void pf_gemm_kernel(PfGemmArgs a) {
 //
 // Workgroups run row tile by row tile on one XCD (token tiles innermost), so that the weights
 // cross HBM once.
+//
+// Measured against the 128-token tiles, whose 96-192 workgroups each walked the whole K: q4, 307
+// rows, hi + lo: gate|up 60 -> 40 us, down 65 -> 26, QKV 26 -> 20, O 25 -> 17; q8, 41 rows (padded
+// to 128 there): 65 -> 16, 85 -> 13, 37 -> 10, 32 -> 9.  The loop runs at the rate of its products
+// (33 of gate|up's 40 us with the products alone, at the clock that they leave); the rest is the
+// first stage's arrival, ~3 us, the exchange and the stores, ~2-3 us.
 template <int FMT, int K, int EPI, int TB, int HL, int WN>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void pf_split_kernel(PfGemmArgs a) {
     constexpr int WK = 8 / WN, NG = K / 64, NKS = K / 32, NXB = (NG + 31) / 32;
@@ -818,13 +824,14 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         __syncthreads();  // every operand read is done (no load is in flight)
 #pragma unroll
         for (int p = 0; p < WK; ++p) {
+            if (part != p) continue;  // one straight run of writes per part
 #pragma unroll
-            for (int i = 0; i < UW; ++i) {
-                const int u = p * UW + i;
-                if (p == part)
-                    sum[i] = acc[u / 4][u % 4];
+            for (int u = 0; u < UN; ++u) {
+                const int own = u / UW;
+                if (own == p)
+                    sum[u % UW] = acc[u / 4][u % 4];
                 else
-                    red[(size_t)(u * (WK - 1) + (part < p ? part : part - 1)) * 64] = acc[u / 4][u % 4];
+                    red[(u * (WK - 1) + (p < own ? p : p - 1)) * 64] = acc[u / 4][u % 4];
             }
         }
         __syncthreads();
@@ -851,13 +858,26 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         const int tq = (tb1 + i / 4) * 16, rb = rb0 + (UW < 4 ? r1 + i : i % 4);
         const float4 tsv = *(const float4*)(a.ts + tq + 4 * q);
         const float tsc[4] = {tsv.x, tsv.y, tsv.z, tsv.w};
+        float y[4];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const float y = sum[i][e] * (tsc[e] * UNBIAS);
-            if (EPI == EPI_STORE || a.splits > 1)
-                __builtin_amdgcn_raw_buffer_store_b32(as_u32(y), drs, ((tq + 4 * q + e) * a.N + rb * 16 + r16) * 4, 0, 0);
-            else
-                pf_store<EPI>(a, tq + 4 * q + e, rb * 16 + r16, y);
+        for (int e = 0; e < 4; ++e) y[e] = sum[i][e] * (tsc[e] * UNBIAS);
+        if (EPI == EPI_STORE || a.splits > 1) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                __builtin_amdgcn_raw_buffer_store_b32(as_u32(y[e]), drs, ((tq + 4 * q + e) * a.N + rb * 16 + r16) * 4, 0, 0);
+        } else if constexpr (EPI == EPI_SWIGLU) {
+            // Lanes r16 < 8 hold gate rows, r16 ^ 8 their up rows: the first take tokens 4 q, 4 q + 1, the
+            // second 4 q + 2, 4 q + 3, so that every lane has two units.
+            const bool lo = r16 < 8;
+            const float o0 = dpp<0x128>(lo ? y[2] : y[0]), o1 = dpp<0x128>(lo ? y[3] : y[1]);
+            const float h0 = lo ? swiglu(y[0], o0) : swiglu(o0, y[2]), h1 = lo ? swiglu(y[1], o1) : swiglu(o1, y[3]);
+            const int t = tq + 4 * q + (lo ? 0 : 2);
+            float* h = a.h + (size_t)t * FF + rb * 8 + (r16 & 7);
+            if (t < a.M) h[0] = h0;
+            if (t + 1 < a.M) h[FF] = h1;
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) pf_store<EPI>(a, tq + 4 * q + e, rb * 16 + r16, y[e]);
         }
     }
 }
@@ -1310,8 +1330,8 @@ static hipError_t pf_split_fmt(int K, int epi, const PfGemmArgs& a, hipStream_t 
                        : pf_split_shape<FMT, 4, 2, 4>(K, epi, a, s);
 }
 
-int pf_gemm_splits(int fmt, int K, int N, int M) {
-    if (!pf_use_split(M)) return 1;
+int pf_gemm_splits(int fmt, int parts, int K, int N, int M) {
+    if (!pf_use_split(fmt, parts, M)) return 1;
     const PfSplitShape t = pf_split_tile(fmt, K, M);
     const int tiles = ((M + 16 * t.tb - 1) / (16 * t.tb)) * (N / (64 * t.wn));
     const int most = std::max(1, std::min(t.nit, 256 / tiles));
@@ -1322,8 +1342,8 @@ int pf_gemm_splits(int fmt, int K, int N, int M) {
 hipError_t launch_pf_gemm(int fmt, int K, int epi, const PfGemmArgs& a, hipStream_t s) {
     if (a.M < 1 || a.N % 256 || (a.parts != 1 && a.parts != 2) || a.splits < 1 || (a.splits > 1 && !a.part))
         return hipErrorInvalidValue;
-    if (pf_use_split(a.M)) {
-        if (a.splits != pf_gemm_splits(fmt, K, a.N, a.M) || a.Mpad < (a.M + 63) / 64 * 64) return hipErrorInvalidValue;
+    if (pf_use_split(fmt, a.parts, a.M)) {
+        if (a.splits != pf_gemm_splits(fmt, a.parts, K, a.N, a.M) || a.Mpad < (a.M + 63) / 64 * 64) return hipErrorInvalidValue;
         switch (fmt) {
             case FMT_Q4: return pf_split_fmt<FMT_Q4>(K, epi, a, s);
             case FMT_Q8: return pf_split_fmt<FMT_Q8>(K, epi, a, s);

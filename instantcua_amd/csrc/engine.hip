@@ -88,18 +88,37 @@ void mrope_table(int maxctx, int vis_offset, int llm_h, int llm_w, std::vector<f
 
 constexpr int PF_CHUNK = 4096;  // rows per matrix-core prefill chunk
 
-struct NullState {
-    State* d = nullptr;
-};
-NullState g_null_state;  // control block for standalone kernels (done = 0)
+// Control block of the standalone kernels: all zero (done = 0; their row count is an argument), in
+// a copy per device.  With the split sums and arrival counters of a K = 6144 product of 2-8 rows
+// (zero between launches; standalone products run on the null stream, one after the other).
+__device__ State g_null_state;
+constexpr int GEMV_SPLIT_ROWS = 4096;
+__device__ float g_gemv_kpart[3 * MAXM * GEMV_SPLIT_ROWS];
+__device__ int g_gemv_kcnt[GEMV_SPLIT_ROWS / 16];
 
-int null_state(State** out, int n) {
-    if (!g_null_state.d) HIPCK(hipMalloc(&g_null_state.d, sizeof(State)));
-    State s{};
-    s.n = n;
-    s.maxctx = 1;
-    HIPCK(hipMemcpy(g_null_state.d, &s, sizeof s, hipMemcpyHostToDevice));
-    *out = g_null_state.d;
+// Their addresses on the current device, looked up once per device.
+struct Standalone {
+    State* st;
+    float* kpart;
+    int* kcnt;
+};
+int standalone_buffers(Standalone& out) {
+    static std::mutex mu;
+    static std::vector<std::pair<int, Standalone>> known;
+    int dev = 0;
+    HIPCK(hipGetDevice(&dev));
+    std::lock_guard<std::mutex> lk(mu);
+    for (const auto& k : known)
+        if (k.first == dev) {
+            out = k.second;
+            return 0;
+        }
+    Standalone b{};
+    HIPCK(hipGetSymbolAddress((void**)&b.st, HIP_SYMBOL(g_null_state)));
+    HIPCK(hipGetSymbolAddress((void**)&b.kpart, HIP_SYMBOL(g_gemv_kpart)));
+    HIPCK(hipGetSymbolAddress((void**)&b.kcnt, HIP_SYMBOL(g_gemv_kcnt)));
+    known.emplace_back(dev, b);
+    out = b;
     return 0;
 }
 
@@ -199,8 +218,7 @@ struct icua_engine {
         return 0;
     }
     int write_state(const State& s) {
-        HIPCK(hipMemcpyAsync(st, &s, sizeof s, hipMemcpyHostToDevice, stream));
-        HIPCK(hipStreamSynchronize(stream));
+        HIPCK(launch_set_state(st, s, stream));
         return 0;
     }
 
@@ -1292,12 +1310,14 @@ int icua_verify(icua_engine* e, const int32_t* draft, int m, int32_t* out_argmax
     for (int l = 0; l < e->layers; ++l)
         if (e->enqueue_layer(l, MAXM, 0)) return -1;
     if (e->enqueue_head(MAXM, 1)) return -1;
-    HIPCK(hipStreamSynchronize(e->stream));
-    HIPCK(hipMemcpy(out_argmax, e->argmax_rows, sizeof(int32_t) * m, hipMemcpyDeviceToHost));
+    if (e->write_state(s)) return -1;
+    // Copies on the pass's own stream, waited for together.
+    HIPCK(hipMemcpyAsync(out_argmax, e->argmax_rows, sizeof(int32_t) * m, hipMemcpyDeviceToHost, e->stream));
     if (out_logits)
-        HIPCK(hipMemcpy(out_logits, e->logits, sizeof(float) * (size_t)m * VOCAB, hipMemcpyDeviceToHost));
+        HIPCK(hipMemcpyAsync(out_logits, e->logits, sizeof(float) * (size_t)m * VOCAB, hipMemcpyDeviceToHost, e->stream));
+    HIPCK(hipStreamSynchronize(e->stream));
     e->last_logits_rows = m;
-    return e->write_state(s);
+    return 0;
 }
 
 int icua_set_position(icua_engine* e, int pos, int32_t next_token, int step, int max_steps) {
@@ -1386,15 +1406,14 @@ static int kv_copy(icua_engine* e, int layer, int kind, int slot0, int nslots, v
     if (layer < 0 || layer >= e->layers || kind < 0 || kind > 1) return fail("bad layer/kind");
     if (slot0 < 0 || nslots < 0 || slot0 + nslots > e->maxctx) return fail("slots out of range");
     if (to_dev && nslots > 0) e->kv_written_from(slot0);
-    for (int g = 0; g < NKV; ++g) {
-        uint16_t* dev = e->kv_ptr(layer, kind) + ((size_t)g * e->maxctx + slot0) * HD;
-        uint16_t* hp = (uint16_t*)host + (size_t)g * nslots * HD;
-        const size_t bytes = (size_t)nslots * HD * 2;
-        if (to_dev)
-            HIPCK(hipMemcpy(dev, hp, bytes, hipMemcpyHostToDevice));
-        else
-            HIPCK(hipMemcpy(hp, dev, bytes, hipMemcpyDeviceToHost));
-    }
+    if (nslots == 0) return 0;
+    // The KV groups' slot ranges in one strided copy.
+    uint16_t* dev = e->kv_ptr(layer, kind) + (size_t)slot0 * HD;
+    const size_t row = (size_t)nslots * HD * 2, pitch = (size_t)e->maxctx * HD * 2;
+    if (to_dev)
+        HIPCK(hipMemcpy2D(dev, pitch, host, row, row, NKV, hipMemcpyHostToDevice));
+    else
+        HIPCK(hipMemcpy2D(host, row, dev, pitch, row, NKV, hipMemcpyDeviceToHost));
     return 0;
 }
 
@@ -1458,10 +1477,14 @@ static int gemv_setup(int fmt, int N, int K, int m, GemvArgs& a, GemvOp& op) {
     if (K != H && K != FF) return fail("K must be 2048 or 6144");
     if (N <= 0 || N % 16) return fail("N must be a positive multiple of 16");
     if (m < 1 || m > MAXM) return fail("m must be 1..8");
-    State* st;
-    if (null_state(&st, m)) return -1;
+    Standalone b;
+    if (standalone_buffers(b)) return -1;
     a = GemvArgs{};
-    a.st = st;
+    a.st = b.st;
+    if (N <= GEMV_SPLIT_ROWS) {
+        a.kpart = b.kpart;
+        a.kcnt = b.kcnt;
+    }
     a.m_fixed = m;
     a.N = N;
     op = (K == H) ? GEMV_PLAIN : GEMV_PLAIN_K6144;

@@ -538,8 +538,10 @@ template <int FMT, int K, int PRO, int EPI>
 static hipError_t launch(const GemvArgs& a, hipStream_t s) {
     const int nrb = EPI == EPI_SWIGLU ? FF / 8 : a.N / 16;
     if constexpr (K == FF && PRO == PRO_F32 && (EPI == EPI_RESID || EPI == EPI_STORE)) {
-        // The engine's partial buffers hold [3][MAXM][H] sums and H / 16 counters.
-        if (a.kpart && a.kcnt && a.N == H) {
+        // With buffers of [3][MAXM][N] sums and N / 16 counters (the engine's, N = 2048; a standalone
+        // product's up to one row block a CU, where walking the three segments in one workgroup
+        // serialises three memory round trips).
+        if (a.kpart && a.kcnt) {
             hipLaunchKernelGGL((gemv8_split_kernel<FMT, EPI>), dim3(nrb * (K / SEG)), dim3(THREADS), 0, s, a);
             return hipGetLastError();
         }

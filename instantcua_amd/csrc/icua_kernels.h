@@ -100,6 +100,8 @@ struct EmbedArgs {
 };
 hipError_t launch_embed(const EmbedArgs& a, hipStream_t s);
 
+// Writes the control block on the stream.
+hipError_t launch_set_state(State* st, const State& v, hipStream_t s);
 // Sets pos / n / logits_rows of the control block on the stream.
 hipError_t launch_set_pass(State* st, int pos, int n, int logits_rows, hipStream_t s);
 

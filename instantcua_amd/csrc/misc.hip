@@ -158,6 +158,17 @@ __global__ void set_pass_kernel(State* st, int pos, int n, int logits_rows) {
     }
 }
 
+// The whole control block, written on the stream from a kernel argument: a copy from host memory
+// waits for the stream.
+__global__ void set_state_kernel(State* st, State v) {
+    if (threadIdx.x == 0) *st = v;
+}
+
+hipError_t launch_set_state(State* st, const State& v, hipStream_t s) {
+    hipLaunchKernelGGL(set_state_kernel, dim3(1), dim3(64), 0, s, st, v);
+    return hipGetLastError();
+}
+
 hipError_t launch_set_pass(State* st, int pos, int n, int logits_rows, hipStream_t s) {
     hipLaunchKernelGGL(set_pass_kernel, dim3(1), dim3(64), 0, s, st, pos, n, logits_rows);
     return hipGetLastError();

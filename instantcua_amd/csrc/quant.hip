@@ -5,13 +5,18 @@
 //
 // q8 (quantizeQ8, 215-241): four elements per lane; the 8 lanes of a group find its maximum with
 // shuffles (max is exact in any order), derive the scale and write their own codes.
-// q4 (quantizeQ4Raw / quantGroup, 243-320): one lane per 64-group, the group in registers.  The
-// lane runs the reference's 5 x 5 clip grid: codes and one least-squares refit of (s, b), fp16
-// rounding of both, the squared error of the rounded pair; the first candidate of least error
-// wins.  The reference's second refit iteration only recomputes codes that the error pass
-// overwrites, so it is not run.  When no candidate is accepted (every fp16 scale rounds to 0) the
-// reference leaves the codes of the chunk's previous group in its code array; a second kernel
-// copies them, so the output bytes match as well (the dequantised values are 0 either way).
+// q4 (quantizeQ4Raw / quantGroup, 243-320): the reference's 5 x 5 clip grid, codes and one
+// least-squares refit of (s, b) per candidate, fp16 rounding of both, the squared error of the
+// rounded pair; the first candidate of least error wins.  The work is bound by vector instructions
+// (about 20 a value and candidate): codes are rounded by one conversion, their sums taken from
+// packed codes, and only the winner's codes are packed for storing.  One lane holds a group and
+// tries every candidate; matrices whose groups would not give every SIMD two wavefronts take five
+// lanes per group, one per lower clip (11 % more instructions, five times the wavefronts).  8.4 M
+// weights 115 us (156 with two roundings and a packing per candidate).  The reference's second refit iteration only
+// recomputes codes that the error pass overwrites, so it is not run.  When no candidate is
+// accepted (every fp16 scale rounds to 0) the reference leaves the codes of the chunk's previous
+// group in its code array; a second kernel copies them, so the output bytes match as well (the
+// dequantised values are 0 either way).
 #include <mutex>
 
 #include "icua_device.h"
@@ -51,19 +56,36 @@ __global__ __launch_bounds__(QT) void quant_q8_kernel(const float* __restrict__ 
     }
 }
 
-__device__ __forceinline__ float code_of(float w, float b, float inv) {
+// min(15, max(0, roundf((w - b) * inv))) as an integer, 0 for NaN.  Clamping first gives the same
+// code, and on [0, 15] v_cvt_rpi_i32_f32 (round to nearest, halves up) is roundf.
+__device__ __forceinline__ uint32_t code_of(float w, float b, float inv) {
 #pragma clang fp contract(off)
-    return sw_min(15.0f, sw_max(0.0f, roundf((w - b) * inv)));
+    const float c = __builtin_amdgcn_fmed3f((w - b) * inv, 0.0f, 15.0f);
+    uint32_t q;
+    asm("v_cvt_rpi_i32_f32 %0, %1" : "=v"(q) : "v"(c));
+    return q;
 }
 
+// Eight codes of w[0 .. 7], four bits each, first lowest.
+__device__ __forceinline__ uint32_t pack_codes(const float* w, float b, float inv) {
+    uint32_t word = 0;
+#pragma unroll
+    for (int t = 0; t < 8; ++t) word |= code_of(w[t], b, inv) << (4 * t);  // q[2k] low nibble, q[2k + 1] high
+    return word;
+}
+
+// QL lanes per group (1 or 5), QG = 64 / QL groups per wave (of 5, four lanes idle).
+template <int QL>
 __global__ __launch_bounds__(QT) void quant_q4_kernel(const float* __restrict__ m, int64_t ngroups,
                                                       uint8_t* __restrict__ packed, uint16_t* __restrict__ sb,
                                                       uint8_t* __restrict__ none) {
 #pragma clang fp contract(off)
-    const int64_t gi = (int64_t)blockIdx.x * QT + threadIdx.x;
-    if (gi >= ngroups) return;
+    constexpr int QG = WAVE / QL;
+    const int lane = threadIdx.x % WAVE, sub = lane % QL;
+    const int64_t gi = ((int64_t)blockIdx.x * (QT / WAVE) + threadIdx.x / WAVE) * QG + lane / QL;
+    const bool live = lane < QL * QG && gi < ngroups;
     float w[64];
-    const float4* src = (const float4*)(m + gi * 64);
+    const float4* src = (const float4*)(m + (live ? gi : 0) * 64);
 #pragma unroll
     for (int k = 0; k < 16; ++k) {
         const float4 v = src[k];
@@ -78,12 +100,12 @@ __global__ __launch_bounds__(QT) void quant_q4_kernel(const float* __restrict__ 
         mn = sw_min(mn, w[i]);
         mx = sw_max(mx, w[i]);
     }
-    uint32_t best[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    uint16_t best_s = 0, best_b = 0;
-    bool accepted = false;
+    uint32_t best = 0;  // fp16 (scale, bias) of the best candidate
+    bool accepted = false, constant = false;
+    float best_err = __builtin_inff();
     if (mx - mn < 1e-12f) {  // constant group: codes 0, (0, mn)
-        best_b = f2h(mn);
-        accepted = true;
+        best = (uint32_t)f2h(mn) << 16;
+        accepted = constant = true;
     } else {
         // The reference accumulates Σw inside every candidate's loop; the sequence is the same
         // each time, so one in-order sum gives the same value.
@@ -92,66 +114,100 @@ __global__ __launch_bounds__(QT) void quant_q4_kernel(const float* __restrict__ 
         for (int i = 0; i < 64; ++i) sw += w[i];
         const float clips[5] = {0.0f, 0.03f, 0.06f, 0.1f, 0.15f};
         const float range = mx - mn;
-        float best_err = __builtin_inff();
-        for (int ai = 0; ai < 5; ++ai) {
-            for (int cj = 0; cj < 5; ++cj) {
-                const float lo = mn + clips[ai] * range, hi = mx - clips[cj] * range;
-                if (hi <= lo) continue;
-                float s = (hi - lo) / 15.0f, b = lo;
-                {
-                    const float inv = 1.0f / s;
-                    float sq = 0.0f, sqq = 0.0f, sqw = 0.0f;
-#pragma unroll
-                    for (int i = 0; i < 64; ++i) {
-                        const float v = code_of(w[i], b, inv);
-                        sq += v;
-                        sqq += v * v;
-                        sqw += v * w[i];
-                    }
-                    const float den = 64.0f * sqq - sq * sq;
-                    if (den > 0.0f) {
-                        const float s2 = (64.0f * sqw - sq * sw) / den;
-                        if (s2 > 0.0f) {
-                            s = s2;
-                            b = (sw - s2 * sq) / 64.0f;
-                        }
-                    }
-                }
-                const uint16_t sh = f2h(s), bh = f2h(b);
-                const float sf = h2f(sh), bf = h2f(bh);
-                if (sf <= 0.0f) continue;
-                const float inv = 1.0f / sf;
-                float err = 0.0f;
-                uint32_t cur[8];
+        for (int c = 0; c < 25 / QL; ++c) {
+            const int ai = QL == 5 ? sub : c / 5, cj = QL == 5 ? c : c % 5;
+            const float ca = ai == 0 ? clips[0] : ai == 1 ? clips[1] : ai == 2 ? clips[2] : ai == 3 ? clips[3] : clips[4];
+            const float cc = cj == 0 ? clips[0] : cj == 1 ? clips[1] : cj == 2 ? clips[2] : cj == 3 ? clips[3] : clips[4];
+            const float lo = mn + ca * range, hi = mx - cc * range;
+            if (hi <= lo) continue;
+            float s = (hi - lo) / 15.0f, b = lo;
+            {
+                // Σq and Σq² are whole numbers below 2^24: exact in any order, taken from the packed codes.
+                const float inv = 1.0f / s;
+                uint32_t iq = 0, iqq = 0;
+                float sqw = 0.0f;
 #pragma unroll
                 for (int j = 0; j < 8; ++j) {
                     uint32_t word = 0;
 #pragma unroll
                     for (int t = 0; t < 8; ++t) {
-                        const int i = 8 * j + t;
-                        const float v = code_of(w[i], bf, inv);
-                        word |= (uint32_t)v << (4 * t);  // q[2k] low nibble, q[2k + 1] high
-                        const float d = sf * v + bf - w[i];
-                        err += d * d;
+                        const uint32_t q = code_of(w[8 * j + t], b, inv);
+                        word |= q << (4 * t);
+                        sqw += (float)q * w[8 * j + t];
                     }
-                    cur[j] = word;
+                    iq = __builtin_amdgcn_udot8(word, 0x11111111u, iq, false);
+                    iqq = __builtin_amdgcn_udot8(word, word, iqq, false);
                 }
-                if (err < best_err) {
-                    best_err = err;
-                    best_s = sh;
-                    best_b = bh;
+                const float sq = (float)iq, sqq = (float)iqq;
+                const float den = 64.0f * sqq - sq * sq;
+                if (den > 0.0f) {
+                    const float s2 = (64.0f * sqw - sq * sw) / den;
+                    if (s2 > 0.0f) {
+                        s = s2;
+                        b = (sw - s2 * sq) / 64.0f;
+                    }
+                }
+            }
+            const uint16_t sh = f2h(s), bh = f2h(b);
+            const float sf = h2f(sh), bf = h2f(bh);
+            if (sf <= 0.0f) continue;
+            const float inv = 1.0f / sf;
+            float err = 0.0f;
 #pragma unroll
-                    for (int j = 0; j < 8; ++j) best[j] = cur[j];
-                    accepted = true;
-                }
+            for (int i = 0; i < 64; ++i) {
+                const float d = sf * (float)code_of(w[i], bf, inv) + bf - w[i];
+                err += d * d;
+            }
+            if (err < best_err) {
+                best_err = err;
+                best = (uint32_t)sh | ((uint32_t)bh << 16);
+                accepted = true;
             }
         }
     }
-    uint4* dst = (uint4*)(packed + gi * 32);
-    dst[0] = make_uint4(best[0], best[1], best[2], best[3]);
-    dst[1] = make_uint4(best[4], best[5], best[6], best[7]);
-    *(uint32_t*)(sb + gi * 2) = (uint32_t)best_s | ((uint32_t)best_b << 16);
-    none[gi] = accepted ? 0 : 1;
+    if constexpr (QL > 1) {
+        // The group's first candidate of least error, to all of its lanes.
+        const int l0 = lane - sub;
+        int win = -1;
+        float least = __builtin_inff();
+#pragma unroll
+        for (int i = 0; i < QL; ++i) {
+            const float e = __shfl(best_err, l0 + i);
+            if (__shfl((int)accepted, l0 + i) && (win < 0 || e < least)) {
+                win = i;
+                least = e;
+            }
+        }
+        best = (uint32_t)__shfl((int)best, l0 + max(win, 0));
+        accepted = win >= 0;
+    }
+    if (!live) return;
+    const float bf = h2f((uint16_t)(best >> 16)), inv = 1.0f / h2f((uint16_t)best);
+    const bool zero = constant || !accepted;  // codes 0
+    if constexpr (QL == 1) {
+        uint32_t o[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) o[j] = zero ? 0u : pack_codes(w + 8 * j, bf, inv);
+        uint4* dst = (uint4*)(packed + gi * 32);
+        dst[0] = make_uint4(o[0], o[1], o[2], o[3]);
+        dst[1] = make_uint4(o[4], o[5], o[6], o[7]);
+    } else if (sub < 4) {  // lanes 0 .. 3 of the group: a quarter each, read again
+        float v[16];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const float4 x = src[4 * sub + k];
+            v[4 * k] = x.x;
+            v[4 * k + 1] = x.y;
+            v[4 * k + 2] = x.z;
+            v[4 * k + 3] = x.w;
+        }
+        *(uint2*)(packed + gi * 32 + 8 * sub) =
+            zero ? make_uint2(0u, 0u) : make_uint2(pack_codes(v, bf, inv), pack_codes(v + 8, bf, inv));
+    }
+    if (sub == 0) {
+        *(uint32_t*)(sb + gi * 2) = best;
+        none[gi] = accepted ? 0 : 1;
+    }
 }
 
 // Groups that accepted no candidate take the codes of the nearest previous group of their
@@ -212,11 +268,13 @@ hipError_t launch_quant(int fmt, const float* m, int64_t rows, int64_t cols, voi
     }
     if (fmt != FMT_Q4) return hipErrorInvalidValue;
     const int64_t ng = n / 64;
-    const dim3 grid((unsigned)((ng + QT - 1) / QT));
-    hipLaunchKernelGGL(quant_q4_kernel, grid, dim3(QT), 0, s, m, ng, (uint8_t*)codes, (uint16_t*)sb, none);
+    const bool one = ng >= 2 * 4 * 256 * WAVE;  // two wavefronts for each of the 1024 SIMDs
+    const int per = QT / WAVE * (one ? WAVE : WAVE / 5);  // groups of a workgroup
+    hipLaunchKernelGGL(one ? quant_q4_kernel<1> : quant_q4_kernel<5>, dim3((unsigned)((ng + per - 1) / per)), dim3(QT), 0, s,
+                       m, ng, (uint8_t*)codes, (uint16_t*)sb, none);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(quant_q4_carry_kernel, grid, dim3(QT), 0, s, ng, 64 * (cols / 64), (uint8_t*)codes,
+    hipLaunchKernelGGL(quant_q4_carry_kernel, dim3((unsigned)((ng + QT - 1) / QT)), dim3(QT), 0, s, ng, 64 * (cols / 64), (uint8_t*)codes,
                        (const uint8_t*)none);
     return hipGetLastError();
 }

@@ -240,11 +240,13 @@ struct icua_engine {
     }
 
     // encodeLLMLayer for the rows of the current pass (pos / n from the control block).
-    int enqueue_layer(int l, int mt, int row0) {
+    // (at most rows_max of them; 0: MAXM).
+    int enqueue_layer(int l, int mt, int row0, int rows_max) {
         const LayerW& w = L[l];
         GemvArgs a{};
         a.st = st;
         a.m_fixed = 0;
+        a.rows_max = rows_max;
         // 1. RMSNorm + fused QKV.
         a.w = w.wqkv;
         a.sb = w.wqkv_sb;
@@ -296,9 +298,10 @@ struct icua_engine {
         return 0;
     }
 
-    int enqueue_head(int mt, int verify_only) {
+    int enqueue_head(int mt, int verify_only, int rows_max) {
         GemvArgs a{};
         a.st = st;
+        a.rows_max = rows_max;
         a.w = E;
         a.sb = Esb;
         a.N = VOCAB;
@@ -325,8 +328,8 @@ struct icua_engine {
 
     int enqueue_step(int mt) {
         for (int l = 0; l < layers; ++l)
-            if (enqueue_layer(l, mt, 0)) return -1;
-        return enqueue_head(mt, 0);
+            if (enqueue_layer(l, mt, 0, 0)) return -1;
+        return enqueue_head(mt, 0, 0);
     }
 
     int decode_mt() const { return (flags & ICUA_FLAG_GRAMMAR_PAIRS) ? MAXM : 1; }
@@ -925,7 +928,7 @@ struct icua_engine {
             }
         }
         HIPCK(launch_set_pass(st, start_pos + n - 1, 1, write_logits ? 1 : 0, stream));
-        return enqueue_head(MAXM, 0);
+        return enqueue_head(MAXM, 0, 1);  // the last row
     }
 
     bool use_pf(int n) const { return n > MAXM && !(flags & ICUA_FLAG_PASS_PREFILL); }
@@ -988,9 +991,9 @@ struct icua_engine {
             ea.n = m;
             HIPCK(launch_embed(ea, stream));
             for (int l = 0; l < layers; ++l)
-                if (enqueue_layer(l, MAXM, r0)) return -1;
+                if (enqueue_layer(l, MAXM, r0, m)) return -1;
         }
-        return enqueue_head(MAXM, 0);
+        return enqueue_head(MAXM, 0, n % MAXM ? n % MAXM : MAXM);
     }
 
     int decode_steps(int k, double* ms_out) {
@@ -1308,8 +1311,8 @@ int icua_verify(icua_engine* e, const int32_t* draft, int m, int32_t* out_argmax
     ea.n = m;
     HIPCK(launch_embed(ea, e->stream));
     for (int l = 0; l < e->layers; ++l)
-        if (e->enqueue_layer(l, MAXM, 0)) return -1;
-    if (e->enqueue_head(MAXM, 1)) return -1;
+        if (e->enqueue_layer(l, MAXM, 0, m)) return -1;
+    if (e->enqueue_head(MAXM, 1, m)) return -1;
     if (e->write_state(s)) return -1;
     // Copies on the pass's own stream, waited for together.
     HIPCK(hipMemcpyAsync(out_argmax, e->argmax_rows, sizeof(int32_t) * m, hipMemcpyDeviceToHost, e->stream));
@@ -1395,7 +1398,7 @@ int icua_layer_step(icua_engine* e, int layer, const float* x_in, int n, int pos
     v.vis_offset = -1;
     if (e->write_state(v)) return -1;
     HIPCK(hipMemcpy(e->x, x_in, sizeof(float) * (size_t)n * H, hipMemcpyHostToDevice));
-    if (e->enqueue_layer(layer, n == 1 ? 1 : MAXM, 0)) return -1;
+    if (e->enqueue_layer(layer, n == 1 ? 1 : MAXM, 0, n)) return -1;
     HIPCK(hipStreamSynchronize(e->stream));
     HIPCK(hipMemcpy(x_out, e->x, sizeof(float) * (size_t)n * H, hipMemcpyDeviceToHost));
     return e->write_state(s);

@@ -69,14 +69,17 @@ __device__ __forceinline__ int sum8_token(int lane) { return 4 * ((lane >> 3) & 
 
 // Four consecutive activations (columns 4 tid .. of the segment) of buffer rows 0 .. MAXM - 1.
 // A host-given row count (m_fixed) bounds the rows read (the ones past it repeat its last row);
-// otherwise the buffer holds MAXM rows (the engine's pass buffers).  Every row is staged and
-// multiplied; only the pass's rows are written (an operand row m = 2 t + part feeds output row m
-// of the matrix-core product alone, so a row never touches another row's sums).
-template <int K>
-__device__ __forceinline__ void load_rows(const GemvArgs& a, int seg, float (&v)[MAXM][4]) {
+// otherwise the buffer holds MAXM rows (the engine's pass buffers).  The first NR rows, 4 or 8 by
+// the host's bound on the pass, are staged, and all 8 multiplied; only the pass's rows are written
+// (an operand row m = 2 t + part feeds output row m of the matrix-core product alone, so a row
+// never touches another row's sums, whatever it holds).  Staging is half of such a kernel's life
+// (of ~6 us at K = 2048: 1.2 until its loads are out, 3 until they are staged, 0.8 for the sums and
+// 0.5 to finish), hence the form of four rows (a q4 verify of 4: 1.37 -> 1.21 ms).
+template <int K, int NR>
+__device__ __forceinline__ void load_rows(const GemvArgs& a, int seg, float (&v)[NR][4]) {
     const int k0 = 4 * threadIdx.x;
 #pragma unroll
-    for (int t = 0; t < MAXM; ++t) {
+    for (int t = 0; t < NR; ++t) {
         const int r = a.m_fixed > 0 ? min(t, a.m_fixed - 1) : t;
         const float4 p = *(const float4*)(a.x + (size_t)r * K + seg * SEG + k0);
         v[t][0] = p.x;
@@ -89,14 +92,16 @@ __device__ __forceinline__ void load_rows(const GemvArgs& a, int seg, float (&v)
 // The fp16 hi / lo split of the loaded activations (times the RMSNorm weights wn) in the
 // operand layout, the (token, group) factors, the q4 group sums and, for PRO_NORM, the per-wave
 // sums of squares of each row.  Ends with a barrier.
-template <int FMT, int PRO, int NPART>
-__device__ __forceinline__ void stage(Smem<NPART>& S, const float (&v)[MAXM][4], float4 wn) {
+template <int FMT, int PRO, int NPART, int NR>
+__device__ __forceinline__ void stage(Smem<NPART>& S, const float (&v)[NR][4], float4 wn) {
     const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
     const int k0 = 4 * tid;  // column within the segment
     if constexpr (PRO == PRO_NORM) {
         float ss[MAXM];
 #pragma unroll
         for (int t = 0; t < MAXM; ++t) {
+            ss[t] = 0.f;
+            if (t >= NR) continue;
             float s = v[t][0] * v[t][0];
             s = fmaf(v[t][1], v[t][1], s);
             s = fmaf(v[t][2], v[t][2], s);
@@ -119,7 +124,7 @@ __device__ __forceinline__ void stage(Smem<NPART>& S, const float (&v)[MAXM][4],
     const int j0 = k0 % 8;  // 0 or 4: halves j0 .. j0 + 3 of the lane's 8
     uint8_t* base = (uint8_t*)(S.A + ks * 64) + 16 * 16 * q + j0 * 2;
 #pragma unroll
-    for (int t = 0; t < MAXM; ++t) {
+    for (int t = 0; t < NR; ++t) {
         float x[4], mx = 0.f;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -338,7 +343,7 @@ __device__ __forceinline__ void store_row(const GemvArgs& a, int t, int row, flo
 }
 
 // Row-block streaming form (every op; K = 6144 walks its three segments per batch of blocks).
-template <int FMT, int K, int PRO, int EPI>
+template <int FMT, int K, int PRO, int EPI, int NR>
 __global__ __launch_bounds__(THREADS, 1) void gemv8_kernel(GemvArgs a) {
     constexpr int NSEG = K / SEG;
     // Blocks per batch: K = 6144 holds two per wave (with three segments' operands staged in turn
@@ -352,7 +357,7 @@ __global__ __launch_bounds__(THREADS, 1) void gemv8_kernel(GemvArgs a) {
     const int nb = (nrb - wg + G - 1) / G;  // blocks of this workgroup (the host keeps wg < nrb)
     const Src src = make_src<FMT, K>(a);
     WTile<FMT> wl[DEPTH];
-    float v[MAXM][4];
+    float v[NR][4];
     // Reduction / epilogue role of this thread: block k0 + re of a batch, buffer row rt, row rr.
     const int re = tid / 128, rt = (tid / 16) % MAXM, rr = tid % 16;
     const int tq = 2 * (lane >> 4), r16 = lane & 15;
@@ -365,12 +370,12 @@ __global__ __launch_bounds__(THREADS, 1) void gemv8_kernel(GemvArgs a) {
     if constexpr (NSEG == 1) {
         // The rows, then the first DEPTH blocks, then the staging: none of it waits for the
         // control block (read after the staging's barriers, so the loads stay ahead of it).
-        load_rows<K>(a, 0, v);
+        load_rows<K, NR>(a, 0, v);
         const float4 wn = PRO == PRO_NORM ? *(const float4*)(a.norm_w + 4 * tid) : make_float4(1.f, 1.f, 1.f, 1.f);
 #pragma unroll
         for (int k = 0; k < DEPTH; ++k) wl[k].template load<K>(src, wg + k * G, k < nb, 0, wave, lane);
         pass = read_pass(a);
-        stage<FMT, PRO>(S, v, wn);
+        stage<FMT, PRO, NPART, NR>(S, v, wn);
         ops.load(S, wave, lane);
         if constexpr (PRO == PRO_NORM) {
             float ss = 0.f;
@@ -404,9 +409,9 @@ __global__ __launch_bounds__(THREADS, 1) void gemv8_kernel(GemvArgs a) {
             for (int seg = 0; seg < NSEG; ++seg) {
                 // (The weights are requested after the staging here: with the rows in flight
                 // too, the registers would not hold them.)
-                load_rows<K>(a, seg, v);
+                load_rows<K, NR>(a, seg, v);
                 __syncthreads();  // every wave has read the previous segment's operands
-                stage<FMT, PRO_F32>(S, v, make_float4(1.f, 1.f, 1.f, 1.f));
+                stage<FMT, PRO_F32, NPART, NR>(S, v, make_float4(1.f, 1.f, 1.f, 1.f));
 #pragma unroll
                 for (int k = 0; k < DP; ++k) wl[k].template load<K>(src, wg + (k0 + k) * G, k0 + k < nb, seg, wave, lane);
                 ops.load(S, wave, lane);
@@ -485,18 +490,18 @@ __global__ __launch_bounds__(THREADS, 1) void gemv8_kernel(GemvArgs a) {
 // stores its block's sums of its segment in a.kpart; the third to arrive at the row block's
 // counter adds the three in segment order (the same result whichever arrives last), applies the
 // epilogue and re-arms the counter.
-template <int FMT, int EPI>
+template <int FMT, int EPI, int NR>
 __global__ __launch_bounds__(THREADS, 1) void gemv8_split_kernel(GemvArgs a) {
     constexpr int K = FF, NSEG = K / SEG;
     __shared__ Smem<1> S;
     const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
     const int nrb = a.N / 16, rb = blockIdx.x % nrb, seg = blockIdx.x / nrb;
-    float v[MAXM][4];
-    load_rows<K>(a, seg, v);
+    float v[NR][4];
+    load_rows<K, NR>(a, seg, v);
     WTile<FMT> wt;
     wt.template load<K>(make_src<FMT, K>(a), rb, true, seg, wave, lane);
     const Pass pass = read_pass(a);
-    stage<FMT, PRO_F32>(S, v, make_float4(1.f, 1.f, 1.f, 1.f));
+    stage<FMT, PRO_F32, 1, NR>(S, v, make_float4(1.f, 1.f, 1.f, 1.f));
     Ops<FMT> ops;
     ops.load(S, wave, lane);
     float y2[2];
@@ -534,7 +539,7 @@ __global__ __launch_bounds__(THREADS, 1) void gemv8_split_kernel(GemvArgs a) {
     if (tid == 0) __hip_atomic_store(a.kcnt + rb, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-template <int FMT, int K, int PRO, int EPI>
+template <int FMT, int K, int PRO, int EPI, int NR>
 static hipError_t launch(const GemvArgs& a, hipStream_t s) {
     const int nrb = EPI == EPI_SWIGLU ? FF / 8 : a.N / 16;
     if constexpr (K == FF && PRO == PRO_F32 && (EPI == EPI_RESID || EPI == EPI_STORE)) {
@@ -542,25 +547,25 @@ static hipError_t launch(const GemvArgs& a, hipStream_t s) {
         // product's up to one row block a CU, where walking the three segments in one workgroup
         // serialises three memory round trips).
         if (a.kpart && a.kcnt) {
-            hipLaunchKernelGGL((gemv8_split_kernel<FMT, EPI>), dim3(nrb * (K / SEG)), dim3(THREADS), 0, s, a);
+            hipLaunchKernelGGL((gemv8_split_kernel<FMT, EPI, NR>), dim3(nrb * (K / SEG)), dim3(THREADS), 0, s, a);
             return hipGetLastError();
         }
     }
     const int G = nrb < 256 ? nrb : 256;
-    hipLaunchKernelGGL((gemv8_kernel<FMT, K, PRO, EPI>), dim3(G), dim3(THREADS), 0, s, a);
+    hipLaunchKernelGGL((gemv8_kernel<FMT, K, PRO, EPI, NR>), dim3(G), dim3(THREADS), 0, s, a);
     return hipGetLastError();
 }
 
-template <int FMT>
+template <int FMT, int NR>
 static hipError_t op_fmt(GemvOp op, const GemvArgs& a, hipStream_t s) {
     switch (op) {
-        case GEMV_QKV: return launch<FMT, H, PRO_NORM, EPI_STORE>(a, s);
-        case GEMV_O: return launch<FMT, H, PRO_F32, EPI_RESID>(a, s);
-        case GEMV_GU: return launch<FMT, H, PRO_NORM, EPI_SWIGLU>(a, s);
-        case GEMV_DOWN: return launch<FMT, FF, PRO_F32, EPI_RESID>(a, s);
-        case GEMV_LMHEAD: return launch<FMT, H, PRO_NORM, EPI_ARGMAX>(a, s);
-        case GEMV_PLAIN: return launch<FMT, H, PRO_F32, EPI_STORE>(a, s);
-        case GEMV_PLAIN_K6144: return launch<FMT, FF, PRO_F32, EPI_STORE>(a, s);
+        case GEMV_QKV: return launch<FMT, H, PRO_NORM, EPI_STORE, NR>(a, s);
+        case GEMV_O: return launch<FMT, H, PRO_F32, EPI_RESID, NR>(a, s);
+        case GEMV_GU: return launch<FMT, H, PRO_NORM, EPI_SWIGLU, NR>(a, s);
+        case GEMV_DOWN: return launch<FMT, FF, PRO_F32, EPI_RESID, NR>(a, s);
+        case GEMV_LMHEAD: return launch<FMT, H, PRO_NORM, EPI_ARGMAX, NR>(a, s);
+        case GEMV_PLAIN: return launch<FMT, H, PRO_F32, EPI_STORE, NR>(a, s);
+        case GEMV_PLAIN_K6144: return launch<FMT, FF, PRO_F32, EPI_STORE, NR>(a, s);
     }
     return hipErrorInvalidValue;
 }
@@ -576,7 +581,10 @@ bool gemv8_supports(int fmt, GemvOp op, int N) {
 
 hipError_t launch_gemv8(int fmt, GemvOp op, const GemvArgs& a, hipStream_t s) {
     if (!gemv8_supports(fmt, op, a.N)) return hipErrorInvalidValue;
-    return fmt == FMT_Q4 ? g8::op_fmt<FMT_Q4>(op, a, s) : g8::op_fmt<FMT_Q8>(op, a, s);
+    if (a.rows_max < 0 || a.rows_max > MAXM || a.m_fixed > MAXM) return hipErrorInvalidValue;
+    const int rows = a.m_fixed > 0 ? a.m_fixed : a.rows_max > 0 ? a.rows_max : MAXM;
+    if (rows <= 4) return fmt == FMT_Q4 ? g8::op_fmt<FMT_Q4, 4>(op, a, s) : g8::op_fmt<FMT_Q8, 4>(op, a, s);
+    return fmt == FMT_Q4 ? g8::op_fmt<FMT_Q4, 8>(op, a, s) : g8::op_fmt<FMT_Q8, 8>(op, a, s);
 }
 
 }  // namespace icua

@@ -34,6 +34,7 @@ struct GemvArgs {
     float* logits;          // EPI_ARGMAX optional logits [MAXM][VOCAB]
     const State* st;
     int m_fixed;            // > 0: rows of the pass given by the host, else st->n
+    int rows_max;           // m_fixed == 0: the host's bound on st->n (0: MAXM)
     int blocks;             // isolated GEMV launches: grid size
     float* kpart;           // K = 6144 residual GEMV: per-segment partials [3][MAXM][N]
     int* kcnt;              // and per-row-block arrival counters [N / 16], zero between launches

@@ -149,20 +149,20 @@ struct PfGemmArgs {
     float* part;
 };
 // Chunks of up to this many rows take the K-split GEMM, larger ones the 128-token tiles, by the
-// weights and the operand parts.  The lines lie where the two meet (4 layers and the head, split /
-// 128-token tiles, ms): hi + lo q4 1.30 / 1.31 at 1000 rows, 2.12 / 2.27 at 1536, 2.55 / 2.37 at 2048
-// (q8 2.33 / 2.47 and 2.82 / 2.56); f16 2.71 / 2.77 at 2048 and 5.04 / 5.28 at 4096, ahead at every
-// size (its 128-token tiles are 128 rows wide).  fp16 operands alone: q4 1.30 / 1.36 at 1280,
-// 1.47 / 1.41 at 1536 (f16 1.62 / 1.70, 1.74 / 1.61); q8 0.85 / 0.87 at 512, 1.13 / 1.01 at 768.
+// weights and the operand parts (a chunk has at most 4096).  The lines lie where the two meet (4
+// layers and the head, split / 128-token tiles, ms): hi + lo q4 1.30 / 1.31 at 1000 rows, 2.09 / 2.27
+// at 1536, 2.53 / 2.37 at 2048 (q8 2.28 / 2.47 and 2.80 / 2.56).  fp16 operands alone q8 1.67 / 1.72 at
+// 2048, 2.58 / 2.49 at 3000; q4 1.49 / 1.61 and 2.28 / 2.42, 2.89 / 2.95 at 4096.  f16 weights are
+// ahead at every size (4096 rows: 4.95 / 5.28, fp16 operands 3.22 / 3.29).
 inline int pf_split_rows(int fmt, int parts) {
-    if (parts == 2) return fmt == FMT_F16 ? 4096 : 1536;
-    return fmt == FMT_Q8 ? 512 : 1280;
+    if (fmt == FMT_F16 || (fmt == FMT_Q4 && parts == 1)) return 4096;
+    return parts == 2 ? 1536 : 2048;
 }
 inline bool pf_use_split(int fmt, int parts, int M) { return M <= pf_split_rows(fmt, parts); }
 int pf_gemm_splits(int fmt, int parts, int K, int N, int M);
-// Partials of a GEMM (at most 256 tiles of 64 x 256) or an attention (256 / 8 query
+// Partials of a GEMM (at most 256 tiles of 128 x 256) or an attention (256 / 8 query
 // blocks and splits of 64 rows), floats.
-constexpr size_t PF_PART_FLOATS = (size_t)256 * 64 * 256;
+constexpr size_t PF_PART_FLOATS = (size_t)256 * 128 * 256;
 constexpr size_t PF_PART_ML_FLOATS = (size_t)32 * 64 * NH * 2;
 static_assert(PF_PART_FLOATS >= (size_t)32 * 64 * H, "attention partials");
 // fmt: FMT_Q4 / FMT_Q8 / FMT_F16 (sb unused for f16); epi: EPI_STORE / EPI_RESID / EPI_SWIGLU;

@@ -53,7 +53,25 @@ __device__ __forceinline__ float swiglu(float y, float up) {
 // a residual row, to which the O / down GEMM's K-split partial sums (and DeepStack rows) are
 // added and written back; attention rows, or their key-split partials, merged; SwiGLU rows, or
 // the gate|up GEMM's K-split partials.
-template <int K, int SRC, int HL, bool Q4>
+//
+// What bounds it at a few hundred rows is the chain of memory round trips, so partials are requested
+// several at a time, whatever their count: through a buffer resource that ends with the last one
+// (past it: zeros, no traffic).
+struct Parts {
+    __amdgpu_buffer_rsrc_t rs;
+    __device__ __forceinline__ Parts(const float* p, size_t floats)
+        : rs(__builtin_amdgcn_make_buffer_rsrc((void*)p, (short)0, (int)(floats * 4), 0x00020000)) {}
+    __device__ __forceinline__ float4 load4(int at) const {  // floats at .. at + 3
+        return __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rs, at * 4, 0, 0));
+    }
+    __device__ __forceinline__ float load(int at) const { return as_f32(__builtin_amdgcn_raw_buffer_load_b32(rs, at * 4, 0, 0)); }
+};
+__device__ __forceinline__ void add8(float (&d)[8], const float4& a0, const float4& a1) {
+    d[0] += a0.x; d[1] += a0.y; d[2] += a0.z; d[3] += a0.w;
+    d[4] += a1.x; d[5] += a1.y; d[6] += a1.z; d[7] += a1.w;
+}
+// PARTS: the source has partials.
+template <int K, int SRC, int HL, bool Q4, bool PARTS>
 __global__ __launch_bounds__(256) void pf_prep_kernel(PfPrepArgs a) {
     constexpr int NU = K / 8 / 256;  // units of 8 activations per thread
     constexpr int NKS = K / 32, NXB = (K / 64 + 31) / 32;
@@ -61,11 +79,6 @@ __global__ __launch_bounds__(256) void pf_prep_kernel(PfPrepArgs a) {
     const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
     __shared__ float red[8];
     float v[NU][8];
-    auto add8 = [](float(&d)[8], const float* p) {
-        const float4 a0 = ((const float4*)p)[0], a1 = ((const float4*)p)[1];
-        d[0] += a0.x; d[1] += a0.y; d[2] += a0.z; d[3] += a0.w;
-        d[4] += a1.x; d[5] += a1.y; d[6] += a1.z; d[7] += a1.w;
-    };
 #pragma unroll
     for (int j = 0; j < NU; ++j)
 #pragma unroll
@@ -77,59 +90,108 @@ __global__ __launch_bounds__(256) void pf_prep_kernel(PfPrepArgs a) {
         w1 = ((const float4*)(a.norm_w + tid * 8))[1];
     }
     if (t < a.M) {
-        if (SRC == PF_SRC_ATTN && a.nsplit > 1) {
-            // Merge of the attention's key splits: head tid / 16, dims 8 (tid % 16) .. + 7.
-            const int head = tid >> 4;
+        if constexpr (SRC == PF_SRC_ATTN && PARTS) {
+            // Merge of the attention's key splits (at most 32): head tid / 16, dims 8 (tid % 16) .. + 7.
+            // The head's 16 lanes load a pair of splits' (max, denominator) each and share the weights.
+            const int head = tid >> 4, l16 = lane & 15;
+            const Parts op(a.part, (size_t)a.nsplit * a.M * H);
             const float2* ml = (const float2*)a.part_ml + (size_t)t * NH + head;
-            const size_t mls = (size_t)a.M * NH, os = (size_t)a.M * H;
-            const float* op = a.part + (size_t)t * H + 8 * tid;
-            float m = -__builtin_inff();
-            for (int s = 0; s < a.nsplit; ++s) m = fmaxf(m, ml[s * mls].x);  // finite: each row sees its own key
-            float l = 0.f;
-#pragma unroll 4
-            for (int s = 0; s < a.nsplit; ++s) {
-                const float2 x = ml[s * mls];
-                const float f = x.x == -__builtin_inff() ? 0.f : __builtin_amdgcn_exp2f(x.x - m);
-                const float4 a0 = ((const float4*)(op + s * os))[0], a1 = ((const float4*)(op + s * os))[1];
-                l = fmaf(x.y, f, l);
-                v[0][0] = fmaf(a0.x, f, v[0][0]); v[0][1] = fmaf(a0.y, f, v[0][1]);
-                v[0][2] = fmaf(a0.z, f, v[0][2]); v[0][3] = fmaf(a0.w, f, v[0][3]);
-                v[0][4] = fmaf(a1.x, f, v[0][4]); v[0][5] = fmaf(a1.y, f, v[0][5]);
-                v[0][6] = fmaf(a1.z, f, v[0][6]); v[0][7] = fmaf(a1.w, f, v[0][7]);
+            float2 x[2];
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+                x[i] = l16 + 16 * i < a.nsplit ? ml[(size_t)(l16 + 16 * i) * a.M * NH] : make_float2(-__builtin_inff(), 0.f);
+            float m = fmaxf(x[0].x, x[1].x);  // finite over the splits: each row sees its own key
+            m = fmaxf(m, dpp<DPP_XOR1>(m));
+            m = fmaxf(m, dpp<DPP_XOR2>(m));
+            m = fmaxf(m, dpp<DPP_HALF_MIRROR>(m));
+            m = fmaxf(m, dpp<DPP_MIRROR>(m));
+            const float f0 = __builtin_amdgcn_exp2f(x[0].x - m), f1 = __builtin_amdgcn_exp2f(x[1].x - m);
+            const float l = sum16(fmaf(x[0].y, f0, x[1].y * f1));
+            for (int s0 = 0; s0 < a.nsplit; s0 += 8) {
+                float4 o[8][2];
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    const int at = ((s0 + i) * a.M + t) * H + 8 * tid;
+                    o[i][0] = op.load4(at);
+                    o[i][1] = op.load4(at + 4);
+                }
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    const float f = __shfl(s0 & 16 ? f1 : f0, (lane & 48) + (s0 & 15) + i);
+                    v[0][0] = fmaf(o[i][0].x, f, v[0][0]); v[0][1] = fmaf(o[i][0].y, f, v[0][1]);
+                    v[0][2] = fmaf(o[i][0].z, f, v[0][2]); v[0][3] = fmaf(o[i][0].w, f, v[0][3]);
+                    v[0][4] = fmaf(o[i][1].x, f, v[0][4]); v[0][5] = fmaf(o[i][1].y, f, v[0][5]);
+                    v[0][6] = fmaf(o[i][1].z, f, v[0][6]); v[0][7] = fmaf(o[i][1].w, f, v[0][7]);
+                }
             }
             const float inv = 1.0f / l;
 #pragma unroll
             for (int i = 0; i < 8; ++i) v[0][i] *= inv;
-        } else if (SRC == PF_SRC_SWIGLU && a.nsplit > 1) {
+        } else if constexpr (SRC == PF_SRC_SWIGLU && PARTS) {
             // Units 8 u .. + 7 are row block u of the gate|up GEMM: 8 gate rows, then 8 up rows.
+            const Parts gu(a.part, (size_t)a.nsplit * a.M * GU);
+            float up[NU][8];
+#pragma unroll
+            for (int j = 0; j < NU; ++j)
+#pragma unroll
+                for (int i = 0; i < 8; ++i) up[j][i] = 0.f;
+            for (int s0 = 0; s0 < a.nsplit; s0 += 2) {
+                float4 o[2][NU][4];
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+#pragma unroll
+                    for (int j = 0; j < NU; ++j)
+#pragma unroll
+                        for (int c = 0; c < 4; ++c) o[i][j][c] = gu.load4(((s0 + i) * a.M + t) * GU + (tid + 256 * j) * 16 + 4 * c);
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+#pragma unroll
+                    for (int j = 0; j < NU; ++j) {
+                        add8(v[j], o[i][j][0], o[i][j][1]);
+                        add8(up[j], o[i][j][2], o[i][j][3]);
+                    }
+            }
+#pragma unroll
+            for (int j = 0; j < NU; ++j)
+#pragma unroll
+                for (int i = 0; i < 8; ++i) v[j][i] = swiglu(v[j][i], up[j][i]);
+        } else {
+            float4 x[NU][2];
 #pragma unroll
             for (int j = 0; j < NU; ++j) {
-                float up[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-                const float* p = a.part + (size_t)t * GU + (size_t)(tid + 256 * j) * 16;
-                for (int s = 0; s < a.nsplit; ++s) {
-                    add8(v[j], p + (size_t)s * a.M * GU);
-                    add8(up, p + (size_t)s * a.M * GU + 8);
-                }
-#pragma unroll
-                for (int i = 0; i < 8; ++i) v[j][i] = swiglu(v[j][i], up[i]);
+                const float4* p = (const float4*)(a.src + (size_t)t * K + (tid + 256 * j) * 8);
+                x[j][0] = p[0];
+                x[j][1] = p[1];
             }
-        } else {
-#pragma unroll
-            for (int j = 0; j < NU; ++j) add8(v[j], a.src + (size_t)t * K + (tid + 256 * j) * 8);
-            if (SRC == PF_SRC_RESID && a.nsplit > 0) {
-                const float* p = a.part + (size_t)t * H + tid * 8;
-                float y[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-#pragma unroll 4
-                for (int s = 0; s < a.nsplit; ++s) add8(y, p + (size_t)s * a.M * H);
-#pragma unroll
-                for (int i = 0; i < 8; ++i) v[0][i] += y[i];
-                if (a.ds) {  // DeepStack residual of a visual row (Shaders.swift:696-707)
-                    const int vrow = a.row0 + t - a.vis_offset;
-                    if (a.vis_offset >= 0 && vrow >= 0 && vrow < a.n_vis) add8(v[0], a.ds + (size_t)vrow * H + tid * 8);
+            if constexpr (SRC == PF_SRC_RESID && PARTS) {
+                const Parts rp(a.part, (size_t)a.nsplit * a.M * H);
+                // DeepStack residual of a visual row (Shaders.swift:696-707)
+                const int vrow = a.row0 + t - a.vis_offset;
+                const bool vis = a.ds && a.vis_offset >= 0 && vrow >= 0 && vrow < a.n_vis;
+                float4 d0, d1;
+                if (vis) {
+                    d0 = ((const float4*)(a.ds + (size_t)vrow * H + tid * 8))[0];
+                    d1 = ((const float4*)(a.ds + (size_t)vrow * H + tid * 8))[1];
                 }
+                for (int s0 = 0; s0 < a.nsplit; s0 += 8) {
+                    float4 o[8][2];
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) {
+                        const int at = ((s0 + i) * a.M + t) * H + tid * 8;
+                        o[i][0] = rp.load4(at);
+                        o[i][1] = rp.load4(at + 4);
+                    }
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) add8(v[0], o[i][0], o[i][1]);
+                }
+                add8(v[0], x[0][0], x[0][1]);
+                if (vis) add8(v[0], d0, d1);
                 float4* xo = (float4*)(a.dst + (size_t)t * K + tid * 8);
                 xo[0] = make_float4(v[0][0], v[0][1], v[0][2], v[0][3]);
                 xo[1] = make_float4(v[0][4], v[0][5], v[0][6], v[0][7]);
+            } else {
+#pragma unroll
+                for (int j = 0; j < NU; ++j) add8(v[j], x[j][0], x[j][1]);
             }
         }
     }
@@ -269,23 +331,24 @@ __device__ __forceinline__ void pf_store(const PfGemmArgs& a, int t, int row, fl
 // blocks per wave, RB = 8 or 16 row blocks); wave w owns token blocks 4 TB tm + TB (w % 4) ..
 // against row blocks RB / 2 (w / 4) onwards (RB / 2 row blocks), two waves per SIMD, and takes
 // its row blocks in halves of four per group.  Each 128-K step, the weight chunks of the RB row
-// blocks (q4 one 1 KiB chunk, q8 two, f16 four) become fp16 B operands in LDS once
+// blocks (q4 one 1 KiB chunk, q8 two) become fp16 B operands in LDS once
 // (double-buffered, 64 or 128 KiB) and are shared by the waves; the waves' activation operands
 // stream from global memory straight into registers two 64-K groups ahead.  The launch takes
 // the largest tile (most products per operand byte) whose count still fills the CUs evenly.
 template <int FMT, int K, int EPI, int PG_RB, int TB, int HL>
 __global__ __launch_bounds__(512) void pf_gemm_kernel(PfGemmArgs a) {
     static_assert((PG_RB == 8 || PG_RB == 16) && (TB == 1 || TB == 2), "tile shape");
+    static_assert(FMT == FMT_Q8 || (FMT == FMT_Q4 && HL == 2), "the other prompts take the K-split GEMM");
     constexpr int NHF = PG_RB / 8;         // halves of four row blocks per wave
     constexpr int TR = 16 * PG_RB;         // rows of a tile
     constexpr int NG = K / 64, NKS = K / 32, NC = K / 128;
-    constexpr int CPS = FMT == FMT_Q4 ? 1 : FMT == FMT_Q8 ? 2 : 4;  // 1 KiB chunks per 128-K step
+    constexpr int CPS = FMT == FMT_Q4 ? 1 : 2;  // 1 KiB chunks per 128-K step
     constexpr int NCH = NC * CPS;                                      // chunks per row block
-    // DQ: the B operands are the dequantised weights in fp16 (q4 s q + b, q8 s q: the reference
-    // engine's prefill precision, taken with fp16 operands alone) or the f16 weights themselves,
-    // so the products accumulate straight into the outputs; otherwise q4 / q8 codes are exact
-    // fp16 integers and each group's sums take their scale in an epilogue.
-    constexpr bool DQ = HL == 1 || FMT == FMT_F16;
+    // DQ: the B operands are the dequantised q8 weights s q in fp16 (the reference engine's prefill
+    // precision, taken with fp16 operands alone), so the products accumulate straight into the
+    // outputs; otherwise codes are exact fp16 integers and each group's sums take their scale in an
+    // epilogue.
+    constexpr bool DQ = HL == 1;
     const int TN = a.N / (16 * PG_RB), TM = a.Mpad / (64 * TB), T = TM * TN;
     const int per = (T + 7) / 8;
     const int tile = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);
@@ -306,7 +369,6 @@ __global__ __launch_bounds__(512) void pf_gemm_kernel(PfGemmArgs a) {
     // Thread t < 2 TR loads one scale word per step (stride 2 words): row t % TR of the tile, q4
     // the (scale, bias) half2 of 64-group 2 c + t / TR; q8 the scales of 32-groups
     // 4 c + 2 (t / TR), + 1 (the same word offsets: a q8 row holds K / 64 words of scale pairs).
-    // f16 weights have no scales.
     const uint32_t* vsrc = (const uint32_t*)a.sb + (size_t)(tn * TR + (tid % TR)) * NG + (tid / TR);
     constexpr int vstride = 2;
     const bool vload = !DQ && (2 * TR >= 512 || tid < 2 * TR);
@@ -343,7 +405,7 @@ __global__ __launch_bounds__(512) void pf_gemm_kernel(PfGemmArgs a) {
 #pragma unroll
             for (int j = 0; j < CPS; ++j) Wn[hb][j] = *(const uint4*)(wsrc + hb * WSRC2 + (size_t)(c * CPS + j) * 1024);
         if (vload) Vn = vsrc[(size_t)c * vstride];
-        if constexpr (DQ && FMT != FMT_F16) {
+        if constexpr (DQ) {
 #pragma unroll
             for (int hb = 0; hb < NHF; ++hb)
 #pragma unroll
@@ -355,10 +417,7 @@ __global__ __launch_bounds__(512) void pf_gemm_kernel(PfGemmArgs a) {
 #pragma unroll
         for (int hb = 0; hb < NHF; ++hb) {
             const int sr = srb + 8 * hb;
-            if constexpr (FMT == FMT_F16) {  // chunk j is k-step j
-#pragma unroll
-                for (int j = 0; j < 4; ++j) Bs[b][sr][j][lane] = Wn[hb][j];
-            } else if constexpr (FMT == FMT_Q8) {
+            if constexpr (FMT == FMT_Q8) {
                 // Bytes 0-7 of a lane of chunk j are k-step 2 j, bytes 8-15 k-step 2 j + 1.
 #pragma unroll
                 for (int j = 0; j < 2; ++j) {
@@ -383,12 +442,6 @@ __global__ __launch_bounds__(512) void pf_gemm_kernel(PfGemmArgs a) {
                 for (int j = 0; j < 4; ++j) {
                     f16x2 o[4];
                     unpack_q4(dd[j], o);
-                    if constexpr (DQ) {  // 64-group 2 c + j / 2: (scale, bias); one rounding each, fma in fp16
-                        const f16x2 sbw = as_h2(Dn[hb][j >> 1]);
-                        const f16x2 sc2 = {sbw.x, sbw.x}, bi2 = {sbw.y, sbw.y};
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) o[i] = __builtin_elementwise_fma(o[i], sc2, bi2);
-                    }
                     Bs[b][sr][j][lane] = pack4(o);
                 }
             }
@@ -893,12 +946,28 @@ __global__ __launch_bounds__(256) void pf_qk_kernel(PfQkArgs a) {
     const int slot = a.p0 + t;
     // The vector's two elements of this lane (vectors are q heads, k groups, v groups in row order),
     // the sum of the QKV GEMM's K-split partials.
-    const float* row = a.qkv + (size_t)t * QKV + vec * HD + lane;
-    float x0 = row[0], x1 = row[64];
-#pragma unroll 4
-    for (int s = 1; s < a.nsplit; ++s) {
-        x0 += row[(size_t)s * a.M * QKV];
-        x1 += row[(size_t)s * a.M * QKV + 64];
+    float x0, x1;
+    if (a.nsplit == 1) {
+        const float* row = a.qkv + (size_t)t * QKV + vec * HD + lane;
+        x0 = row[0];
+        x1 = row[64];
+    } else {
+        const Parts qp(a.qkv, (size_t)a.nsplit * a.M * QKV);
+        x0 = x1 = 0.f;
+        for (int s0 = 0; s0 < a.nsplit; s0 += 8) {
+            float y[8][2];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const int at = ((s0 + i) * a.M + t) * QKV + vec * HD + lane;
+                y[i][0] = qp.load(at);
+                y[i][1] = qp.load(at + 64);
+            }
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                x0 += y[i][0];
+                x1 += y[i][1];
+            }
+        }
     }
     const float* cs = a.rope + (size_t)slot * 128;
     if (vec < NH) {
@@ -1218,17 +1287,17 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 
 // ------------------------------------------------------------------------------------------
 
-template <int K, int SRC>
+template <int K, int SRC, bool PARTS>
 static hipError_t pf_prep_src(int fmt, const PfPrepArgs& a, hipStream_t s) {
     const dim3 grid(a.Mpad), block(256);
     if (a.parts == 2 && fmt == FMT_Q4)
-        hipLaunchKernelGGL((pf_prep_kernel<K, SRC, 2, true>), grid, block, 0, s, a);
+        hipLaunchKernelGGL((pf_prep_kernel<K, SRC, 2, true, PARTS>), grid, block, 0, s, a);
     else if (a.parts == 2)
-        hipLaunchKernelGGL((pf_prep_kernel<K, SRC, 2, false>), grid, block, 0, s, a);
+        hipLaunchKernelGGL((pf_prep_kernel<K, SRC, 2, false, PARTS>), grid, block, 0, s, a);
     else if (fmt == FMT_Q4)
-        hipLaunchKernelGGL((pf_prep_kernel<K, SRC, 1, true>), grid, block, 0, s, a);
+        hipLaunchKernelGGL((pf_prep_kernel<K, SRC, 1, true, PARTS>), grid, block, 0, s, a);
     else
-        hipLaunchKernelGGL((pf_prep_kernel<K, SRC, 1, false>), grid, block, 0, s, a);
+        hipLaunchKernelGGL((pf_prep_kernel<K, SRC, 1, false, PARTS>), grid, block, 0, s, a);
     return hipGetLastError();
 }
 
@@ -1237,9 +1306,13 @@ hipError_t launch_pf_prep(int fmt, int src, const PfPrepArgs& a, hipStream_t s) 
         (a.nsplit > 0 && !a.part))
         return hipErrorInvalidValue;
     switch (src) {
-        case PF_SRC_RESID: return pf_prep_src<H, PF_SRC_RESID>(fmt, a, s);
-        case PF_SRC_ATTN: return pf_prep_src<H, PF_SRC_ATTN>(fmt, a, s);
-        case PF_SRC_SWIGLU: return pf_prep_src<FF, PF_SRC_SWIGLU>(fmt, a, s);
+        case PF_SRC_RESID:
+            return a.nsplit > 0 ? pf_prep_src<H, PF_SRC_RESID, true>(fmt, a, s) : pf_prep_src<H, PF_SRC_RESID, false>(fmt, a, s);
+        case PF_SRC_ATTN:
+            if (a.nsplit > 32) return hipErrorInvalidValue;
+            return a.nsplit > 1 ? pf_prep_src<H, PF_SRC_ATTN, true>(fmt, a, s) : pf_prep_src<H, PF_SRC_ATTN, false>(fmt, a, s);
+        case PF_SRC_SWIGLU:
+            return a.nsplit > 1 ? pf_prep_src<FF, PF_SRC_SWIGLU, true>(fmt, a, s) : pf_prep_src<FF, PF_SRC_SWIGLU, false>(fmt, a, s);
     }
     return hipErrorInvalidValue;
 }
@@ -1251,7 +1324,7 @@ hipError_t launch_pf_last_row(const PfPrepArgs& a, int t, hipStream_t s) {
 }
 
 template <int FMT, int RB, int TB, int HL>
-static hipError_t pf_gemm_shape_hl(int K, int epi, const PfGemmArgs& a, hipStream_t s) {
+static hipError_t pf_gemm_shape(int K, int epi, const PfGemmArgs& a, hipStream_t s) {
     const int T = (a.Mpad / (64 * TB)) * (a.N / (16 * RB));
     const dim3 grid(8 * ((T + 7) / 8));
     if (K == H && epi == EPI_STORE)
@@ -1267,27 +1340,19 @@ static hipError_t pf_gemm_shape_hl(int K, int epi, const PfGemmArgs& a, hipStrea
     return hipGetLastError();
 }
 
-template <int FMT, int RB, int TB>
-static hipError_t pf_gemm_shape(int K, int epi, const PfGemmArgs& a, hipStream_t s) {
-    return a.parts == 1 ? pf_gemm_shape_hl<FMT, RB, TB, 1>(K, epi, a, s) : pf_gemm_shape_hl<FMT, RB, TB, 2>(K, epi, a, s);
-}
-
 // Tiles that fill the 256 CUs evenly: at least one each, and a whole number each or at least four.
 static bool even_fill(int tiles) { return tiles >= 256 && (tiles % 256 == 0 || tiles >= 1024); }
 
 // The largest tile whose count fills the CUs evenly: 128 tokens x 256 rows, 128 x 128, else
-// 64 x 128 (small prompts, whose 128-token tiles would leave CUs idle).  f16 weights keep 128-row
-// tiles (their four B chunks per step would not fit the registers of the larger tile), and so do
-// fp16 operands alone: their 128-row tile needs ~110 registers and 64 KiB of LDS, so two
+// 64 x 128.  fp16 operands alone keep 128-row tiles: their 128-row tile needs ~110 registers and 64 KiB of LDS, so two
 // workgroups share a CU (measured 21.55 -> 20.97 ms per 4096-row prefill against 256-row tiles).
-template <int FMT>
+template <int FMT, int HL>
 static hipError_t pf_gemm_fmt(int K, int epi, const PfGemmArgs& a, hipStream_t s) {
     const int tm128 = a.Mpad / 128;
-    if (FMT != FMT_F16 && a.parts == 2 && a.N % 256 == 0 && even_fill(tm128 * (a.N / 256))) {
-        if constexpr (FMT != FMT_F16) return pf_gemm_shape<FMT, 16, 2>(K, epi, a, s);
-    }
-    if (even_fill(tm128 * (a.N / 128))) return pf_gemm_shape<FMT, 8, 2>(K, epi, a, s);
-    return pf_gemm_shape<FMT, 8, 1>(K, epi, a, s);
+    if constexpr (HL == 2)
+        if (even_fill(tm128 * (a.N / 256))) return pf_gemm_shape<FMT, 16, 2, HL>(K, epi, a, s);
+    if (even_fill(tm128 * (a.N / 128))) return pf_gemm_shape<FMT, 8, 2, HL>(K, epi, a, s);
+    return pf_gemm_shape<FMT, 8, 1, HL>(K, epi, a, s);
 }
 
 template <int FMT, int TB, int HL, int WN>
@@ -1308,21 +1373,31 @@ static hipError_t pf_split_shape(int K, int epi, const PfGemmArgs& a, hipStream_
 }
 
 // Tiles of the K-split GEMM: 32 tokens (two token blocks) up to 32 rows, else 64; 128 weight rows
-// while there is one token tile, else 256 (a tile's operands are then shared by four row groups).
+// while there is one token tile, and for O and down (N = 2048) up to four, where the partials of
+// twice the splits would cost more than the operands of twice the tiles (q4 at 128 rows 0.461 /
+// 0.483 ms, 4 layers and the head; 0.590 / 0.616 at 256, 0.657 / 0.654 at 307), else 256 (a tile's
+// operands are then shared by four row groups).
+// With fp16 operands alone there are half the products per unpacked weight, and the unpacking bounds
+// a 64-token tile: 128 tokens from the size on where that pays (4 layers and the head, 128 / 64
+// tokens, ms): q8 0.57 / 0.59 at 256 rows, 1.04 / 1.21 at 1000; f16 0.69 / 0.74 at 384, 0.62 / 0.60 at
+// 256; q4 1.08 / 1.28 at 1280, 0.93 / 0.89 at 1000.
 struct PfSplitShape {
     int tb, wn, nit;  // token blocks, row groups, iterations of K
 };
-static PfSplitShape pf_split_tile(int fmt, int K, int M) {
-    const int tb = M <= 32 ? 2 : 4, wn = M <= 64 ? 2 : 4;
+static int pf_wide_rows(int fmt) { return fmt == FMT_Q8 ? 192 : fmt == FMT_F16 ? 320 : 1152; }
+static PfSplitShape pf_split_tile(int fmt, int parts, int K, int N, int M) {
+    const int tb = M <= 32 ? 2 : parts == 1 && M >= pf_wide_rows(fmt) ? 8 : 4;
+    const int wn = M <= 64 || (M <= 256 && N == H && tb == 4) ? 2 : 4;
     const int unit = fmt == FMT_Q4 && wn == 4 ? 128 : 64;
     return {tb, wn, K / (8 / wn * unit)};
 }
 
 template <int FMT>
 static hipError_t pf_split_fmt(int K, int epi, const PfGemmArgs& a, hipStream_t s) {
-    const PfSplitShape t = pf_split_tile(FMT, K, a.M);
+    const PfSplitShape t = pf_split_tile(FMT, a.parts, K, a.N, a.M);
     if (a.parts == 1)
         return t.tb == 2   ? pf_split_shape<FMT, 2, 1, 2>(K, epi, a, s)
+               : t.tb == 8 ? pf_split_shape<FMT, 8, 1, 4>(K, epi, a, s)
                : t.wn == 2 ? pf_split_shape<FMT, 4, 1, 2>(K, epi, a, s)
                            : pf_split_shape<FMT, 4, 1, 4>(K, epi, a, s);
     return t.tb == 2   ? pf_split_shape<FMT, 2, 2, 2>(K, epi, a, s)
@@ -1332,7 +1407,7 @@ static hipError_t pf_split_fmt(int K, int epi, const PfGemmArgs& a, hipStream_t 
 
 int pf_gemm_splits(int fmt, int parts, int K, int N, int M) {
     if (!pf_use_split(fmt, parts, M)) return 1;
-    const PfSplitShape t = pf_split_tile(fmt, K, M);
+    const PfSplitShape t = pf_split_tile(fmt, parts, K, N, M);
     const int tiles = ((M + 16 * t.tb - 1) / (16 * t.tb)) * (N / (64 * t.wn));
     const int most = std::max(1, std::min(t.nit, 256 / tiles));
     const int its = (t.nit + most - 1) / most;
@@ -1343,7 +1418,7 @@ hipError_t launch_pf_gemm(int fmt, int K, int epi, const PfGemmArgs& a, hipStrea
     if (a.M < 1 || a.N % 256 || (a.parts != 1 && a.parts != 2) || a.splits < 1 || (a.splits > 1 && !a.part))
         return hipErrorInvalidValue;
     if (pf_use_split(fmt, a.parts, a.M)) {
-        if (a.splits != pf_gemm_splits(fmt, a.parts, K, a.N, a.M) || a.Mpad < (a.M + 63) / 64 * 64) return hipErrorInvalidValue;
+        if (a.splits != pf_gemm_splits(fmt, a.parts, K, a.N, a.M) || a.Mpad < (a.M + 63) / 64 * 64 || (a.parts == 1 && a.Mpad % 128 && a.M > 64)) return hipErrorInvalidValue;
         switch (fmt) {
             case FMT_Q4: return pf_split_fmt<FMT_Q4>(K, epi, a, s);
             case FMT_Q8: return pf_split_fmt<FMT_Q8>(K, epi, a, s);
@@ -1352,12 +1427,9 @@ hipError_t launch_pf_gemm(int fmt, int K, int epi, const PfGemmArgs& a, hipStrea
         return hipErrorInvalidValue;
     }
     if (a.Mpad < a.M || a.Mpad % 128 || a.splits != 1) return hipErrorInvalidValue;
-    switch (fmt) {
-        case FMT_Q4: return pf_gemm_fmt<FMT_Q4>(K, epi, a, s);
-        case FMT_Q8: return pf_gemm_fmt<FMT_Q8>(K, epi, a, s);
-        case FMT_F16: return pf_gemm_fmt<FMT_F16>(K, epi, a, s);
-    }
-    return hipErrorInvalidValue;
+    if (fmt == FMT_Q8) return a.parts == 2 ? pf_gemm_fmt<FMT_Q8, 2>(K, epi, a, s) : pf_gemm_fmt<FMT_Q8, 1>(K, epi, a, s);
+    if (fmt == FMT_Q4 && a.parts == 2) return pf_gemm_fmt<FMT_Q4, 2>(K, epi, a, s);
+    return hipErrorInvalidValue;  // pf_split_rows sends every other chunk the other way
 }
 
 hipError_t launch_pf_qk(const PfQkArgs& a, hipStream_t s) {

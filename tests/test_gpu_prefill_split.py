@@ -66,10 +66,12 @@ def test_split_prefill_matches_passes(fmt, n, start):
     check(image(fmt), synth.random_tokens(start + n, f"split-{n}-{start}"), start)
 
 
-@pytest.mark.parametrize("fmt,n", [("q4", 1536), ("q4", 1537), ("q8", 513), ("f16", 1281)])
+# hi + lo: the last size of four 64-token tiles (O and down change their width), of the K-split GEMM
+# and one past each.  fp16 operands: the first sizes of the 128-token tiles of the K-split GEMM (q8
+# 192, f16 320, q4 1152) and the first past it (q8 2049).
+@pytest.mark.parametrize("fmt,n", [("q4", 256), ("q8", 257), ("q4", 1536), ("q4", 1537), ("q8", 191), ("q8", 192),
+                                   ("f16", 320), ("q4", 1152), ("q8", 2049)])
 def test_sizes_where_the_tiles_change_match_passes(fmt, n):
-    """The last size of the K-split GEMM and the first of the 128-token tiles (hi + lo q4; fp16
-    operands q8 and f16)."""
     check(image(fmt), synth.random_tokens(n, f"split-{n}"))
 
 

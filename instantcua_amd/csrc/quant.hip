@@ -12,11 +12,11 @@
 // packed codes, and only the winner's codes are packed for storing.  One lane holds a group and
 // tries every candidate; matrices whose groups would not give every SIMD two wavefronts take five
 // lanes per group, one per lower clip (11 % more instructions, five times the wavefronts).  8.4 M
-// weights 115 us (156 with two roundings and a packing per candidate).  The reference's second refit iteration only
-// recomputes codes that the error pass overwrites, so it is not run.  When no candidate is
-// accepted (every fp16 scale rounds to 0) the reference leaves the codes of the chunk's previous
-// group in its code array; a second kernel copies them, so the output bytes match as well (the
-// dequantised values are 0 either way).
+// weights 115 us (156 with two roundings and a packing per candidate), 0.5 M 29 us (131).  The
+// reference's second refit iteration only recomputes codes that the error pass overwrites, so it
+// is not run.  When no candidate is accepted (every fp16 scale rounds to 0) the reference leaves the
+// codes of the chunk's previous group in its code array; a second kernel copies them, so the output
+// bytes match as well (the dequantised values are 0 either way).
 #include <mutex>
 
 #include "icua_device.h"

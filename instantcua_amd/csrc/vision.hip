@@ -90,10 +90,41 @@ __device__ __forceinline__ void dma_barrier() {
     asm volatile("" ::: "memory");
 }
 
+// 0.5 x (1 + tanh(u)) = x / (1 + exp(-2 u)), u = sqrt(2 / pi) (x + 0.044715 x^3): one v_exp and one
+// v_rcp (tanhf made the epilogue of fc1 half as long as its loop).
 __device__ __forceinline__ float gelu_tanh(float x) {
-    return 0.5f * x * (1.0f + tanhf(0.7978845608028654f * (x + 0.044715f * x * x * x)));
+    const float u = 0.7978845608028654f * (x + 0.044715f * x * x * x);
+    return x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-2.0f * 1.4426950408889634f * u));
 }
 __device__ __forceinline__ float gelu_erf(float x) { return 0.5f * x * (1.0f + erff(x * 0.7071067811865475f)); }
+
+// Four consecutive outputs n .. n + 3 of token m: bias and the mode's elementwise work.
+template <int MODE>
+__device__ __forceinline__ void vit_store(const VitGemmArgs& g, int m, int n, const f32x4& acc) {
+#pragma clang fp contract(off)
+    const float4 bv = *(const float4*)(g.bias + n);
+    float4 v = make_float4(acc[0] + bv.x, acc[1] + bv.y, acc[2] + bv.z, acc[3] + bv.w);
+    const size_t o = (size_t)m * g.N + n;
+    if constexpr (MODE == VG_F32) {
+        *(float4*)(g.outf + o) = v;
+    } else if constexpr (MODE == VG_F32_ADD) {
+        float4 r = *(const float4*)(g.outf + o);
+        r.x += v.x;
+        r.y += v.y;
+        r.z += v.z;
+        r.w += v.w;
+        *(float4*)(g.outf + o) = r;
+    } else if constexpr (MODE == VG_F32_POS) {
+        const float4 p = *(const float4*)(g.pos + o);
+        *(float4*)(g.outf + o) = make_float4(v.x + p.x, v.y + p.y, v.z + p.z, v.w + p.w);
+    } else {
+        float e[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) e[i] = MODE == VG_GELU_TANH ? gelu_tanh(e[i]) : gelu_erf(e[i]);
+        const uint32_t h0 = f2h(e[0]), h1 = f2h(e[1]), h2 = f2h(e[2]), h3 = f2h(e[3]);
+        *(uint2*)(g.outh + o) = make_uint2(h0 | (h1 << 16), h2 | (h3 << 16));
+    }
+}
 
 // C[m][n] = sum_k X[m][k] W[n][k] over fp16 X [M][K] and W [N][K].  Workgroup tile BN x BM
 // (outputs x tokens), 4 waves in a WN x WM grid; each wave holds TN x TM 16 x 16 accumulators.
@@ -105,8 +136,12 @@ __device__ __forceinline__ float gelu_erf(float x) { return 0.5f * x * (1.0f + e
 // holds 128-byte rows; the 16-byte chunk c of row r sits at chunk c ^ (r % 8), so the 16 rows
 // of a fragment read spread over the banks.  Token rows past M read row M - 1 and are not
 // stored.
-template <int BN, int BM, int WN, int WM, int MODE, int S = 4>
-__global__ __launch_bounds__(256) void vit_gemm_kernel(VitGemmArgs g) {
+//
+// (The launch bound is twice the 256 threads that run: a wave then has at most 256 registers, all of
+// them VGPRs.  With more, the compiler keeps the accumulators in AGPRs and moves them to and fro
+// around every few products.)
+template <int BN, int BM, int WN, int WM, int MODE, int S>
+__global__ __launch_bounds__(512) void vit_gemm_kernel(VitGemmArgs g) {
 #pragma clang fp contract(off)
     constexpr int TN = BN / WN / 16, TM = BM / WM / 16, BK = 64;
     constexpr int WLOADS = (BN + BM) / 8;  // 1 KiB wave loads per stage (8 rows each)
@@ -166,7 +201,6 @@ __global__ __launch_bounds__(256) void vit_gemm_kernel(VitGemmArgs g) {
     }
     __builtin_amdgcn_s_waitcnt(0);  // no load is in flight when the workgroup ends
 
-    const int N = g.N;
 #pragma unroll
     for (int b = 0; b < TM; ++b) {
         const int m = m0 + (wm * TM + b) * 16 + r16;
@@ -213,51 +247,145 @@ __global__ __launch_bounds__(256) void vit_gemm_kernel(VitGemmArgs g) {
 #pragma unroll
             for (int a = 0; a < TN; ++a) {
                 const int n = n0 + (wn * TN + a) * 16 + 4 * q4;
-                const float4 bv = *(const float4*)(g.bias + n);
-                float4 v = make_float4(acc[a][b][0] + bv.x, acc[a][b][1] + bv.y, acc[a][b][2] + bv.z, acc[a][b][3] + bv.w);
-                const size_t o = (size_t)m * N + n;
-                if constexpr (MODE == VG_F32) {
-                    *(float4*)(g.outf + o) = v;
-                } else if constexpr (MODE == VG_F32_ADD) {
-                    float4 r = *(const float4*)(g.outf + o);
-                    r.x += v.x;
-                    r.y += v.y;
-                    r.z += v.z;
-                    r.w += v.w;
-                    *(float4*)(g.outf + o) = r;
-                } else if constexpr (MODE == VG_F32_POS) {
-                    const float4 p = *(const float4*)(g.pos + o);
-                    *(float4*)(g.outf + o) = make_float4(v.x + p.x, v.y + p.y, v.z + p.z, v.w + p.w);
-                } else {
-                    float e[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) e[i] = MODE == VG_GELU_TANH ? gelu_tanh(e[i]) : gelu_erf(e[i]);
-                    const uint32_t h0 = f2h(e[0]), h1 = f2h(e[1]), h2 = f2h(e[2]), h3 = f2h(e[3]);
-                    *(uint2*)(g.outh + o) = make_uint2(h0 | (h1 << 16), h2 | (h3 << 16));
-                }
+                vit_store<MODE>(g, m, n, acc[a][b]);
             }
         }
     }
 }
 
+// The same product where few tiles cover the result and K is long (fc2, the mergers, the patch
+// embedding): 64 outputs x 64 tokens per workgroup, 4 waves, each computing the whole tile over its
+// own steps of K (step w, w + 4, ...) through an LDS ring of its own, so no wave waits for another
+// before the end, where their sums meet in LDS.  LDS traffic bounds these products (with four waves
+// sharing a stage as 32 x 32 quarters, 48 KiB a step at 128 bytes a clock): a wave's 64 x 64 tile
+// reads each operand once, 32 KiB a step.  (The launch bound as above.)  At 960 patches fc2 takes
+// 19.6 us and a merger's two products 39.9 (with 32 x 64 tiles over shared stages 22.6 and 53).
+// proj, with four steps of K a wave, would take 9.7 against 8.7: the start and the sums at the end
+// cost more there than the shared stages do.
+template <int MODE>
+__global__ __launch_bounds__(512) void vit_deep_kernel(VitGemmArgs g) {
+#pragma clang fp contract(off)
+    static_assert(MODE != VG_QKV, "the rotation pairs of a head are not in one lane here");
+    constexpr int KW = 4;
+    __shared__ __align__(1024) uint8_t rings[KW][2][128 * 128];  // [wave][stage][64 W rows, 64 X rows][64 K]
+    const int tid = threadIdx.x, lane = tid % WAVE, wave = __builtin_amdgcn_readfirstlane(tid / WAVE), r16 = lane & 15, q4 = lane >> 4;
+    const int n0 = blockIdx.x * 64, m0 = blockIdx.y * 64, K = g.K, nk = K / 64;
+    // As in vit_gemm_kernel: load j brings rows 8 j .. + 7, 16-byte chunk c of row r lands at c ^ (r % 8).
+    const int lrow = lane >> 3, lchunk = (lane & 7) ^ lrow;
+    auto issue = [&](int st, int kt) __attribute__((always_inline)) {
+        const int k0 = kt * 64 + 8 * lchunk;
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+            const uint16_t* src = j < 8 ? g.W + (size_t)(n0 + 8 * j + lrow) * K + k0
+                                        : g.X + (size_t)min(m0 + 8 * (j - 8) + lrow, g.M - 1) * K + k0;
+            __builtin_amdgcn_global_load_lds(src, (__attribute__((address_space(3))) void*)(rings[wave][st] + 1024 * j), 16, 0, 0);
+        }
+    };
+    f32x4 acc[4][4];
+#pragma unroll
+    for (int a = 0; a < 4; ++a)
+#pragma unroll
+        for (int b = 0; b < 4; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // A step's two k-steps alternate between two register sets: while one is multiplied, the other's
+    // operands are read.  Behind the first, the next step's stage has to have landed; behind the
+    // second, the present stage is free for the step after that.
+    struct Ops {
+        v8h w[4], x[4];
+    };
+    auto read = [&](int st, int ks) __attribute__((always_inline)) {
+        const uint8_t* s = rings[wave][st];
+        Ops o;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            const int row = 16 * t + r16, at = row * 128 + (((4 * ks + q4) ^ (row & 7)) << 4);
+            o.w[t] = *(const v8h*)(s + at);
+            o.x[t] = *(const v8h*)(s + 64 * 128 + at);
+        }
+        return o;
+    };
+    auto mac = [&](const Ops& o) __attribute__((always_inline)) {
+#pragma unroll
+        for (int a = 0; a < 4; ++a)
+#pragma unroll
+            for (int b = 0; b < 4; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(o.w[a], o.x[b], acc[a][b], 0, 0, 0);
+    };
+    constexpr int VM0 = (7 << 4) | (15 << 8), VM16 = VM0 | ((16 >> 4) << 14), LGKM0 = 15 | (7 << 4) | (3 << 14);
+    if (wave < nk) {
+        issue(0, wave);
+        if (wave + KW < nk) {
+            issue(1, wave + KW);
+            __builtin_amdgcn_s_waitcnt(VM16);
+        } else {
+            __builtin_amdgcn_s_waitcnt(VM0);
+        }
+        asm volatile("" ::: "memory");
+        Ops p0 = read(0, 0);
+        for (int kt = wave, st = 0; kt < nk; kt += KW, st ^= 1) {
+            const Ops p1 = read(st, 1);
+            __builtin_amdgcn_sched_barrier(0);
+            mac(p0);
+            __builtin_amdgcn_sched_barrier(0);
+            __builtin_amdgcn_s_waitcnt(LGKM0);  // the stage has been read
+            asm volatile("" ::: "memory");
+            if (kt + 2 * KW < nk) {
+                issue(st, kt + 2 * KW);
+                __builtin_amdgcn_s_waitcnt(VM16);
+            } else {
+                __builtin_amdgcn_s_waitcnt(VM0);
+            }
+            asm volatile("" ::: "memory");
+            p0 = read(st ^ 1, 0);  // (after the last step: a stage that is not used)
+            __builtin_amdgcn_sched_barrier(0);
+            mac(p1);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    // Wave w finishes output rows 16 w .. + 15 of the tile (blocks (w, 0 .. 3)), the sums in wave order.
+    __syncthreads();
+    f32x4* sums = (f32x4*)&rings[0][0][0];  // [wave][block][lane], 64 KiB
+#pragma unroll
+    for (int a = 0; a < 4; ++a)
+#pragma unroll
+        for (int b = 0; b < 4; ++b) sums[(wave * 16 + 4 * a + b) * WAVE + lane] = acc[a][b];
+    __syncthreads();
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+        f32x4 y = sums[(4 * wave + b) * WAVE + lane];
+#pragma unroll
+        for (int w = 1; w < KW; ++w) {
+            const f32x4 o = sums[(w * 16 + 4 * wave + b) * WAVE + lane];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) y[e] += o[e];
+        }
+        const int m = m0 + 16 * b + r16;
+        if (m < g.M) vit_store<MODE>(g, m, n0 + 16 * wave + 4 * q4, y);
+    }
+}
+
 // Bidirectional attention of one head over all patches (k_vit_attn, Shaders.swift:294-395),
-// grid (ceil(np / 64), 16 heads), 8 waves.  Waves w and w + 4 own the same 16 queries,
-// 64 x + 16 (w % 4) .. + 15 (lane l: query l % 16), and split the key blocks in two halves, so the
-// serial chain of block loads is half as long.  Per block of 64 keys: S^T = K . Q^T on
-// v_mfma_f32_16x16x32_f16 (lane: keys 16 j + 4 (l / 16) + i of sub-block j), scaled by 1/8; an
-// online softmax per query column; O^T += V^T . P^T on v_mfma_f32_16x16x16_f16 with the fp16
-// probabilities straight from the score registers and V^T read from LDS.  The two halves'
-// (max, sum, O) are combined through LDS.  Keys past np are masked (their rows hold finite
-// values).
-__global__ __launch_bounds__(512) void vit_attention_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
-                                                            const uint16_t* __restrict__ vt, uint16_t* __restrict__ out,
-                                                            int np, int ld) {
-    constexpr int ROW = 72, TILE = 64 * ROW;
-    // [key half][K, V^T][buffer].  V^T rows with (row / 8) odd hold their 4-key chunks pairwise
-    // swapped (chunk c at c ^ 1): the P.V reads of 16 rows x one chunk then cover all 32 banks.
-    __shared__ __align__(16) uint16_t lds[2][2][2][TILE];
+// grid (ceil(np / 64), 16 heads), 16 waves.  Waves w, w + 4, w + 8 and w + 12 own the same 16
+// queries, 64 x + 16 (w % 4) .. + 15 (lane l: query l % 16), and split the key blocks in four, so
+// the serial chain of block loads and softmax updates, which bounds the kernel (the products of
+// 960 patches take ~3 us of it), is a quarter as long.  Per block of 64 keys: S^T = K . Q^T on
+// v_mfma_f32_16x16x32_f16 (lane: keys 16 j + 4 (l / 16) + i of sub-block j), in log2 units
+// (log2(e) / 8, so that every exponential is one v_exp_f32); an online softmax per query column
+// whose denominators stay per lane until the end; O^T += V^T . P^T on v_mfma_f32_16x16x16_f16 with
+// the fp16 probabilities straight from the score registers and V^T read from LDS, rescaled only
+// when some column's maximum moved.  The four parts' (max, sum, O) are combined through LDS.  Keys
+// past np are masked (their rows hold finite values; only the last block has any).  960 patches:
+// 13.4 us; with two key parts, 8 waves and unprefetched V operands 20.8.
+constexpr int VA_PARTS = 4, VA_ROW = 72, VA_TILE = 64 * VA_ROW;
+constexpr size_t VA_LDS = (size_t)VA_PARTS * 2 * 2 * VA_TILE * 2;  // [part][K, V^T][buffer]: 147,456 B
+__global__ __launch_bounds__(1024) void vit_attention_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
+                                                             const uint16_t* __restrict__ vt, uint16_t* __restrict__ out,
+                                                             int np, int ld) {
+    // V^T rows with (row / 8) odd hold their 4-key chunks pairwise swapped (chunk c at c ^ 1): the
+    // P.V reads of 16 rows x one chunk then cover all 32 banks.
+    extern __shared__ __align__(16) uint16_t va_lds[];
     const int tid = threadIdx.x, lane = tid % WAVE, wave = tid / WAVE, r16 = lane & 15, q4 = lane >> 4;
     const int grp = wave >> 2, gt = tid & 255;
+    uint16_t* kt = va_lds + (size_t)grp * 4 * VA_TILE;  // K of buffer 0, 1, then V^T of buffer 0, 1
+    uint16_t* vtl = kt + 2 * VA_TILE;
     const int h = blockIdx.y;
     const int qt = blockIdx.x * 64 + (wave & 3) * 16 + r16;
     const uint16_t* qh = q + (size_t)h * ld * VHD;
@@ -268,125 +396,165 @@ __global__ __launch_bounds__(512) void vit_attention_kernel(const uint16_t* __re
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) qf[ks] = *(const v8h*)(qh + (size_t)qc * VHD + 32 * ks + 8 * q4);
 
-    // Register-staged block loads by the 256 threads of a half (macros: see vit_gemm_kernel).
-    uint4 kr[2], vr[2];
-#define VA_GLOAD(blk_)                                                              \
-    do {                                                                            \
-        _Pragma("unroll") for (int c = 0; c < 2; ++c) {                              \
-            const int idx = gt + 256 * c, row = idx >> 3, col = (idx & 7) * 8;       \
-            kr[c] = *(const uint4*)(kh + (size_t)(64 * (blk_) + row) * VHD + col);   \
-            vr[c] = *(const uint4*)(vh + (size_t)row * ld + 64 * (blk_) + col);      \
-        }                                                                           \
-    } while (0)
-#define VA_LSTORE(buf_)                                                             \
-    do {                                                                            \
-        _Pragma("unroll") for (int c = 0; c < 2; ++c) {                              \
-            const int idx = gt + 256 * c, row = idx >> 3, col = (idx & 7) * 8;       \
-            *(uint4*)&lds[grp][0][buf_][row * ROW + col] = kr[c];                    \
-            const uint4 vv_ = ((row >> 3) & 1) ? make_uint4(vr[c].z, vr[c].w, vr[c].x, vr[c].y) : vr[c]; \
-            *(uint4*)&lds[grp][1][buf_][row * ROW + col] = vv_;                      \
-        }                                                                           \
-    } while (0)
+    // Register-staged block loads by the 256 threads of a part: rows gt / 8 and 32 + gt / 8, columns
+    // 8 (gt % 8) .. + 7.
+    struct Block {
+        uint4 k0, k1, v0, v1;
+    };
+    const int row = gt >> 3, col = (gt & 7) * 8;
+    auto gload = [&](int blk) __attribute__((always_inline)) {
+        const uint16_t* kp = kh + (size_t)(64 * blk + row) * VHD + col;
+        const uint16_t* vp = vh + (size_t)row * ld + 64 * blk + col;
+        return Block{*(const uint4*)kp, *(const uint4*)(kp + 32 * VHD), *(const uint4*)vp, *(const uint4*)(vp + (size_t)32 * ld)};
+    };
+    auto lstore = [&](int buf, const Block& x) __attribute__((always_inline)) {
+        uint16_t* kd = kt + buf * VA_TILE + row * VA_ROW + col;
+        uint16_t* vd = vtl + buf * VA_TILE + row * VA_ROW + col;
+        const bool odd = (row >> 3) & 1;
+        *(uint4*)kd = x.k0;
+        *(uint4*)(kd + 32 * VA_ROW) = x.k1;
+        *(uint4*)vd = odd ? make_uint4(x.v0.z, x.v0.w, x.v0.x, x.v0.y) : x.v0;
+        *(uint4*)(vd + 32 * VA_ROW) = odd ? make_uint4(x.v1.z, x.v1.w, x.v1.x, x.v1.y) : x.v1;
+    };
 
-    const int nblk = (np + 63) / 64, nh = (nblk + 1) / 2;
-    const int b0 = grp * nh, bend = min(nblk, b0 + nh);  // this half's blocks [b0, bend)
-    float m_run = -__builtin_inff(), l_run = 0.f;
+    const int nblk = (np + 63) / 64, nh = (nblk + VA_PARTS - 1) / VA_PARTS;
+    const int b0 = min(nblk, grp * nh), bend = min(nblk, b0 + nh);  // this part's blocks [b0, bend), maybe none
+    float m_run = -__builtin_inff(), l_run = 0.f;  // maximum of query r16; this lane's share of its denominator
     f32x4 O[4];
 #pragma unroll
     for (int dt = 0; dt < 4; ++dt) O[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
-    VA_GLOAD(min(b0, nblk - 1));
-    VA_LSTORE(0);
+    lstore(0, gload(min(b0, nblk - 1)));
     __syncthreads();
     for (int it = 0; it < nh; ++it) {
         const int blk = b0 + it, buf = it & 1;
-        VA_GLOAD(min(blk + 1, nblk - 1));  // unconditional (a valid block either way)
-        if (blk < bend) {
-            const uint16_t* Ks = lds[grp][0][buf];
-            const uint16_t* Vs = lds[grp][1][buf];
+        const Block next = gload(min(blk + 1, nblk - 1));  // a valid block either way
+        {  // (no branch around it: a step past the part's blocks masks every key)
+            const int lim = blk < bend ? np : 0;
+            const uint16_t* Ks = kt + buf * VA_TILE;
+            const uint16_t* Vs = vtl + buf * VA_TILE;
             f32x4 S[4];
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 S[j] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                 for (int ks = 0; ks < 2; ++ks) {
-                    const v8h kf = *(const v8h*)&Ks[(16 * j + r16) * ROW + 32 * ks + 8 * q4];
+                    const v8h kf = *(const v8h*)&Ks[(16 * j + r16) * VA_ROW + 32 * ks + 8 * q4];
                     S[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, qf[ks], S[j], 0, 0, 0);
                 }
+            }
+            // The V operands, read behind the softmax.
+            v4h vf[4][4];
+#pragma unroll
+            for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) vf[dt][j] = *(const v4h*)&Vs[(16 * dt + r16) * VA_ROW + 4 * ((4 * j + q4) ^ (r16 >> 3))];
+            if (64 * blk + 64 > lim) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        if (64 * blk + 16 * j + 4 * q4 + i >= lim) S[j][i] = -__builtin_inff();
             }
             float mb = -__builtin_inff();
 #pragma unroll
             for (int j = 0; j < 4; ++j)
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const int key = 64 * blk + 16 * j + 4 * q4 + i;
-                    S[j][i] = key < np ? S[j][i] * 0.125f : -__builtin_inff();
-                    mb = fmaxf(mb, S[j][i]);
-                }
-            mb = max_x4(mb);  // finite: key 64 blk < np
-            const float m_new = fmaxf(m_run, mb);
-            const float corr = expf(m_run - m_new);
+                for (int i = 0; i < 4; ++i) mb = fmaxf(mb, S[j][i]);
+            constexpr float SC = 0.125f * 1.4426950408889634f;
+            const float m_new = fmaxf(m_run, max_x4(mb) * SC);
+            const float m_use = m_new == -__builtin_inff() ? 0.f : m_new;  // a part without a block yet
+            const float corr = __builtin_amdgcn_exp2f(m_run - m_use);
             float ls = 0.f;
             v4h P[4];
 #pragma unroll
             for (int j = 0; j < 4; ++j)
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    const float p = expf(S[j][i] - m_new);
+                    const float p = __builtin_amdgcn_exp2f(S[j][i] * SC - m_use);
                     ls += p;
                     P[j][i] = (_Float16)p;
                 }
-            l_run = l_run * corr + sum_x4(ls);
+            if (__builtin_amdgcn_ballot_w64(m_new != m_run)) {
+                l_run *= corr;
+#pragma unroll
+                for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) O[dt][i] *= corr;
+            }
+            l_run += ls;
             m_run = m_new;
 #pragma unroll
-            for (int dt = 0; dt < 4; ++dt) {
+            for (int j = 0; j < 4; ++j)
 #pragma unroll
-                for (int i = 0; i < 4; ++i) O[dt][i] *= corr;
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const v4h vf = *(const v4h*)&Vs[(16 * dt + r16) * ROW + 4 * ((4 * j + q4) ^ (r16 >> 3))];
-                    O[dt] = __builtin_amdgcn_mfma_f32_16x16x16f16(vf, P[j], O[dt], 0, 0, 0);
-                }
-            }
+                for (int dt = 0; dt < 4; ++dt) O[dt] = __builtin_amdgcn_mfma_f32_16x16x16f16(vf[dt][j], P[j], O[dt], 0, 0, 0);
         }
-        VA_LSTORE(buf ^ 1);  // the last fills an idle buffer
+        lstore(buf ^ 1, next);  // the last fills an idle buffer
         __syncthreads();
     }
-#undef VA_GLOAD
-#undef VA_LSTORE
-    // Combine the halves: the second half's state goes through LDS (every tile read is done).
-    float* xo = (float*)&lds[0][0][0][0];  // [256 lanes][18]
-    if (grp == 1) {
-        float* d = xo + (size_t)gt * 18;
+    l_run = sum_x4(l_run);
+    // Combine the parts: the states of parts 1 .. 3 go through LDS (every tile read is done) as
+    // [part - 1][O tile, then (max, sum)][256 lanes], and part 0 finishes.
+    f32x4* xo = (f32x4*)va_lds;
+    float2* xm = (float2*)(xo + (size_t)(VA_PARTS - 1) * 4 * 256);
+    if (grp > 0) {
 #pragma unroll
-        for (int dt = 0; dt < 4; ++dt)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) d[4 * dt + i] = O[dt][i];
-        d[16] = m_run;
-        d[17] = l_run;
+        for (int dt = 0; dt < 4; ++dt) xo[((grp - 1) * 4 + dt) * 256 + gt] = O[dt];
+        xm[(grp - 1) * 256 + gt] = make_float2(m_run, l_run);
     }
     __syncthreads();
     if (grp == 0 && qt < np) {
-        const float* d = xo + (size_t)gt * 18;
-        const float m1 = d[16], m = fmaxf(m_run, m1);
-        const float f0 = expf(m_run - m), f1 = expf(m1 - m);  // m is finite: the first half is never empty
-        const float inv = 1.0f / (l_run * f0 + d[17] * f1);
+        float2 ml[VA_PARTS - 1];
+        float m = m_run;  // finite: the first part is never empty
+#pragma unroll
+        for (int p = 0; p < VA_PARTS - 1; ++p) {
+            ml[p] = xm[p * 256 + gt];
+            m = fmaxf(m, ml[p].x);
+        }
+        const float f0 = __builtin_amdgcn_exp2f(m_run - m);
+        float l = l_run * f0;
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) O[dt][i] *= f0;
+#pragma unroll
+        for (int p = 0; p < VA_PARTS - 1; ++p) {
+            const float f = __builtin_amdgcn_exp2f(ml[p].x - m);  // 0 for a part without blocks
+            l = fmaf(ml[p].y, f, l);
+#pragma unroll
+            for (int dt = 0; dt < 4; ++dt) {
+                const f32x4 o = xo[(p * 4 + dt) * 256 + gt];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) O[dt][i] = fmaf(o[i], f, O[dt][i]);
+            }
+        }
+        const float inv = 1.0f / l;
         uint16_t* dst = out + (size_t)qt * VH + h * VHD;
 #pragma unroll
         for (int dt = 0; dt < 4; ++dt) {
-            float o[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) o[i] = (O[dt][i] * f0 + d[4 * dt + i] * f1) * inv;
-            const uint32_t h0 = f2h(o[0]), h1 = f2h(o[1]), h2 = f2h(o[2]), h3 = f2h(o[3]);
+            const uint32_t h0 = f2h(O[dt][0] * inv), h1 = f2h(O[dt][1] * inv), h2 = f2h(O[dt][2] * inv), h3 = f2h(O[dt][3] * inv);
             *(uint2*)(dst + 16 * dt + 4 * q4) = make_uint2(h0 | (h1 << 16), h2 | (h3 << 16));
         }
     }
 }
 
-template <int BN, int BM, int WN, int WM, int MODE, int S = 4>
+hipError_t attention(const VitBuffers& b, int np, hipStream_t s) {
+    hipLaunchKernelGGL(vit_attention_kernel, dim3((np + 63) / 64, VNH), dim3(256 * VA_PARTS), VA_LDS, s, b.q, b.k, b.vt, b.attn,
+                       np, NPATCH_MAX);
+    return hipGetLastError();
+}
+
+template <int BN, int BM, int WN, int WM, int MODE, int S>
 hipError_t gemm(const VitGemmArgs& g, hipStream_t s) {
     if (g.N % BN || g.K % 64 || g.M < 1) return hipErrorInvalidValue;
     const dim3 grid(g.N / BN, (g.M + BM - 1) / BM);
     hipLaunchKernelGGL((vit_gemm_kernel<BN, BM, WN, WM, MODE, S>), grid, dim3(256), 0, s, g);
+    return hipGetLastError();
+}
+
+template <int MODE>
+hipError_t gemm_deep(const VitGemmArgs& g, hipStream_t s) {
+    if (g.N % 64 || g.K % 64 || g.M < 1) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(vit_deep_kernel<MODE>, dim3(g.N / 64, (g.M + 63) / 64), dim3(256), 0, s, g);
     return hipGetLastError();
 }
 
@@ -411,7 +579,7 @@ hipError_t merger(const VitMerger& mg, const uint16_t* xn, int nvis, uint16_t* h
     g.M = nvis;
     g.N = MH;
     g.K = MH;
-    VCK((gemm<32, 64, 2, 2, VG_GELU_ERF>(g, s)));
+    VCK((gemm_deep<VG_GELU_ERF>(g, s)));
     g = VitGemmArgs{};
     g.X = hbuf;
     g.W = mg.fc2w;
@@ -420,7 +588,7 @@ hipError_t merger(const VitMerger& mg, const uint16_t* xn, int nvis, uint16_t* h
     g.M = nvis;
     g.N = H;
     g.K = MH;
-    return gemm<32, 32, 2, 2, VG_F32>(g, s);
+    return gemm_deep<VG_F32>(g, s);
 }
 
 }  // namespace
@@ -428,6 +596,7 @@ hipError_t merger(const VitMerger& mg, const uint16_t* xn, int nvis, uint16_t* h
 hipError_t launch_vision(const VitWeights& w, const VitBuffers& b, int gh, int gw, hipStream_t s) {
     const int np = gh * gw, nvis = np / 4;
     if (gh < 2 || gw < 2 || gh % 2 || gw % 2 || np > NPATCH_MAX) return hipErrorInvalidValue;
+    VCK(hipFuncSetAttribute((const void*)vit_attention_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)VA_LDS));
     hipLaunchKernelGGL(vit_patchify_kernel, dim3(np), dim3(256), 0, s, b.rgb, b.patches, gh, gw);
     VCK(hipGetLastError());
     VitGemmArgs g{};
@@ -439,7 +608,7 @@ hipError_t launch_vision(const VitWeights& w, const VitBuffers& b, int gh, int g
     g.M = np;
     g.N = VH;
     g.K = VPATCH;
-    VCK((gemm<32, 64, 2, 2, VG_F32_POS>(g, s)));
+    VCK((gemm_deep<VG_F32_POS>(g, s)));
     int ds = 0;
     for (int l = 0; l < VLAYERS; ++l) {
         const VitBlock& L = w.blk[l];
@@ -456,10 +625,9 @@ hipError_t launch_vision(const VitWeights& w, const VitBuffers& b, int gh, int g
         g.M = np;
         g.N = VQKV;
         g.K = VH;
-        VCK((gemm<64, 64, 1, 4, VG_QKV>(g, s)));
-        hipLaunchKernelGGL(vit_attention_kernel, dim3((np + 63) / 64, VNH), dim3(512), 0, s, b.q, b.k, b.vt, b.attn, np,
-                           NPATCH_MAX);
-        VCK(hipGetLastError());
+        // (a head's 64 outputs x 128 tokens: 15.7 us for 960 patches, 64 x 64 tiles 18.9)
+        VCK((gemm<64, 128, 1, 4, VG_QKV, 3>(g, s)));
+        VCK(attention(b, np, s));
         g = VitGemmArgs{};
         g.X = b.attn;
         g.W = L.projw;
@@ -468,7 +636,7 @@ hipError_t launch_vision(const VitWeights& w, const VitBuffers& b, int gh, int g
         g.M = np;
         g.N = VH;
         g.K = VH;
-        VCK((gemm<32, 64, 2, 2, VG_F32_ADD>(g, s)));
+        VCK((gemm<32, 64, 2, 2, VG_F32_ADD, 4>(g, s)));
         VCK(layernorm<VH>(b.x, L.n2w, L.n2b, b.xn, np, s));
         g = VitGemmArgs{};
         g.X = b.xn;
@@ -478,6 +646,7 @@ hipError_t launch_vision(const VitWeights& w, const VitBuffers& b, int gh, int g
         g.M = np;
         g.N = VFF;
         g.K = VH;
+        // (16.2 us; 64 x 64 tiles 20.1, 128 x 128 tiles, too few of them, 19.8)
         VCK((gemm<128, 64, 2, 2, VG_GELU_TANH, 3>(g, s)));
         g = VitGemmArgs{};
         g.X = b.h;
@@ -487,7 +656,7 @@ hipError_t launch_vision(const VitWeights& w, const VitBuffers& b, int gh, int g
         g.M = np;
         g.N = VH;
         g.K = VFF;
-        VCK((gemm<32, 64, 2, 2, VG_F32_ADD>(g, s)));
+        VCK((gemm_deep<VG_F32_ADD>(g, s)));
         if (l == 5 || l == 11 || l == 17) {
             // DeepStack merger: LayerNorm over each 2 x 2 block's 4096 values (Engine.swift:420-447).
             VCK(layernorm<MH>(b.x, w.mg[ds].nw, w.mg[ds].nb, b.xn, nvis, s));

@@ -1,0 +1,29 @@
+"""GPU parity of the vision tower at patch counts where its work splits have remainders: fewer
+patches than a tile, one more than a 64-patch block, and key blocks that leave parts of the
+attention with fewer blocks than the others or none (1, 2, 3 and 5 blocks over four parts)."""
+import numpy as np
+import pytest
+
+from instantcua_amd import synth
+from instantcua_amd.engine import Engine
+from instantcua_amd.modelfile import WeightFormat
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def vimg():
+    return synth.build_model_image(WeightFormat.Q4, n_layers=1, tag="q4-vision", vision=True)
+
+
+@pytest.mark.parametrize("gh,gw", [(2, 2), (2, 34), (10, 14), (10, 26)])
+def test_tower_matches_oracle_at_remainders(oracle_mod, vimg, gh, gw):
+    rgb = synth.random_rgb(gh, gw, "edges", 100 * gh + gw)
+    ref_p, ref_ds = oracle_mod.vision(vimg, rgb)
+    with Engine(flags=0, image=vimg, max_context=64, max_steps=4) as e:
+        for _ in range(2):  # the second pass over buffers that hold the first one's rows
+            e.vision(rgb)
+            p, ds = e.visual_rows()
+            for got, ref in zip([p, *ds], [ref_p, *ref_ds]):
+                # the same fp16 rounding points, float32 sums in another order: the bar of the tower's tests
+                assert float(np.abs(got - ref).max() / np.abs(ref).max()) < 1e-2

@@ -259,7 +259,7 @@ __global__ __launch_bounds__(512) void vit_gemm_kernel(VitGemmArgs g) {
 // before the end, where their sums meet in LDS.  LDS traffic bounds these products (with four waves
 // sharing a stage as 32 x 32 quarters, 48 KiB a step at 128 bytes a clock): a wave's 64 x 64 tile
 // reads each operand once, 32 KiB a step.  (The launch bound as above.)  At 960 patches fc2 takes
-// 19.6 us and a merger's two products 39.9 (with 32 x 64 tiles over shared stages 22.6 and 53).
+// 19.6 us and a merger's two products 39.9 (with 32-output tiles over shared stages 22.2 and 45.4).
 // proj, with four steps of K a wave, would take 9.7 against 8.7: the start and the sums at the end
 // cost more there than the shared stages do.
 template <int MODE>
@@ -625,7 +625,8 @@ hipError_t launch_vision(const VitWeights& w, const VitBuffers& b, int gh, int g
         g.M = np;
         g.N = VQKV;
         g.K = VH;
-        // (a head's 64 outputs x 128 tokens: 15.7 us for 960 patches, 64 x 64 tiles 18.9)
+        // (a head's 64 outputs x 128 tokens: 15.7 us for 960 patches; x 64 tokens 18.6, x 192 15.6,
+        // x 256 19.3)
         VCK((gemm<64, 128, 1, 4, VG_QKV, 3>(g, s)));
         VCK(attention(b, np, s));
         g = VitGemmArgs{};
@@ -646,7 +647,7 @@ hipError_t launch_vision(const VitWeights& w, const VitBuffers& b, int gh, int g
         g.M = np;
         g.N = VFF;
         g.K = VH;
-        // (16.2 us; 64 x 64 tiles 20.1, 128 x 128 tiles, too few of them, 19.8)
+        // (16.2 us; 19.8 with the accumulators in AGPRs; 128 x 128 tiles, one a CU, 18.9)
         VCK((gemm<128, 64, 2, 2, VG_GELU_TANH, 3>(g, s)));
         g = VitGemmArgs{};
         g.X = b.h;

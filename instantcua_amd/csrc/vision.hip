@@ -253,15 +253,16 @@ __global__ __launch_bounds__(512) void vit_gemm_kernel(VitGemmArgs g) {
     }
 }
 
-// The same product where few tiles cover the result and K is long (fc2, the mergers, the patch
-// embedding): 64 outputs x 64 tokens per workgroup, 4 waves, each computing the whole tile over its
-// own steps of K (step w, w + 4, ...) through an LDS ring of its own, so no wave waits for another
-// before the end, where their sums meet in LDS.  LDS traffic bounds these products (with four waves
-// sharing a stage as 32 x 32 quarters, 48 KiB a step at 128 bytes a clock): a wave's 64 x 64 tile
-// reads each operand once, 32 KiB a step.  (The launch bound as above.)  At 960 patches fc2 takes
-// 19.6 us and a merger's two products 39.9 (with 32-output tiles over shared stages 22.2 and 45.4).
-// proj, with four steps of K a wave, would take 9.7 against 8.7: the start and the sums at the end
-// cost more there than the shared stages do.
+// The same product where K is long and there are 64 x 64 tiles for most of the chip, but not for more
+// of it than once (fc2, the mergers' first product): 64 outputs x 64 tokens per workgroup, 4 waves,
+// each computing the whole tile over its own steps of K (step w, w + 4, ...) through an LDS ring of
+// its own, so no wave waits for another before the end, where their sums meet in LDS.  LDS traffic
+// bounds these products (with four waves sharing a stage as 32 x 32 quarters, 48 KiB a step at 128
+// bytes a clock): a wave's 64 x 64 tile reads each operand once, 32 KiB a step.  (The launch bound
+// as above.)  At 960 patches fc2 takes 19.6 us and a merger's first product 21.4 (with 32 x 64 tiles
+// over shared stages 22.2 and 27.6).  Small tiles with shared stages stay better where K is short
+// (proj 8.7 against 9.7, the patch embedding 9.4 against 9.9) or 64 x 64 tiles fill half of the chip
+// (a merger's second product, 17.8 against 18.5).
 template <int MODE>
 __global__ __launch_bounds__(512) void vit_deep_kernel(VitGemmArgs g) {
 #pragma clang fp contract(off)
@@ -588,7 +589,7 @@ hipError_t merger(const VitMerger& mg, const uint16_t* xn, int nvis, uint16_t* h
     g.M = nvis;
     g.N = H;
     g.K = MH;
-    return gemm_deep<VG_F32>(g, s);
+    return gemm<32, 32, 2, 2, VG_F32, 4>(g, s);
 }
 
 }  // namespace
@@ -608,7 +609,7 @@ hipError_t launch_vision(const VitWeights& w, const VitBuffers& b, int gh, int g
     g.M = np;
     g.N = VH;
     g.K = VPATCH;
-    VCK((gemm_deep<VG_F32_POS>(g, s)));
+    VCK((gemm<32, 64, 2, 2, VG_F32_POS, 4>(g, s)));
     int ds = 0;
     for (int l = 0; l < VLAYERS; ++l) {
         const VitBlock& L = w.blk[l];

@@ -253,16 +253,16 @@ __global__ __launch_bounds__(512) void vit_gemm_kernel(VitGemmArgs g) {
     }
 }
 
-// The same product where K is long and there are 64 x 64 tiles for most of the chip, but not for more
-// of it than once (fc2, the mergers' first product): 64 outputs x 64 tokens per workgroup, 4 waves,
-// each computing the whole tile over its own steps of K (step w, w + 4, ...) through an LDS ring of
-// its own, so no wave waits for another before the end, where their sums meet in LDS.  LDS traffic
-// bounds these products (with four waves sharing a stage as 32 x 32 quarters, 48 KiB a step at 128
-// bytes a clock): a wave's 64 x 64 tile reads each operand once, 32 KiB a step.  (The launch bound
-// as above.)  At 960 patches fc2 takes 19.6 us and a merger's first product 21.4 (with 32 x 64 tiles
-// over shared stages 22.2 and 27.6).  Small tiles with shared stages stay better where K is short
-// (proj 8.7 against 9.7, the patch embedding 9.4 against 9.9) or 64 x 64 tiles fill half of the chip
-// (a merger's second product, 17.8 against 18.5).
+// The same product where K is long and there are more 32 x 64 tiles than CUs (fc2 and the mergers'
+// first product; gemm_long): 64 outputs x 64 tokens per workgroup, 4 waves, each computing the whole
+// tile over its own steps of K (step w, w + 4, ...) through an LDS ring of its own, so no wave waits
+// for another before the end, where their sums meet in LDS.  LDS traffic bounds these products (with
+// four waves sharing a stage as 32 x 32 quarters, 48 KiB a step at 128 bytes a clock): a wave's 64 x
+// 64 tile reads each operand once, 32 KiB a step.  (The launch bound as above.)  At 960 patches fc2
+// takes 19.0 us and a merger's first product 20.8 (with 32 x 64 tiles over shared stages 21.2 and
+// 26.7).  Small tiles with shared stages stay better where K is short (proj 8.7 against 9.7, the patch
+// embedding 9.4 against 9.9) or 64 x 64 tiles fill half of the chip (a merger's second product, 17.8
+// against 18.5).
 template <int MODE>
 __global__ __launch_bounds__(512) void vit_deep_kernel(VitGemmArgs g) {
 #pragma clang fp contract(off)
@@ -364,20 +364,23 @@ __global__ __launch_bounds__(512) void vit_deep_kernel(VitGemmArgs g) {
 }
 
 // Bidirectional attention of one head over all patches (k_vit_attn, Shaders.swift:294-395),
-// grid (ceil(np / 64), 16 heads), 16 waves.  Waves w, w + 4, w + 8 and w + 12 own the same 16
-// queries, 64 x + 16 (w % 4) .. + 15 (lane l: query l % 16), and split the key blocks in four, so
+// grid (ceil(np / 64), 16 heads), 4 PARTS waves.  Waves w, w + 4, .. own the same 16 queries,
+// 64 x + 16 (w % 4) .. + 15 (lane l: query l % 16), and split the key blocks in PARTS parts, so
 // the serial chain of block loads and softmax updates, which bounds the kernel (the products of
-// 960 patches take ~3 us of it), is a quarter as long.  Per block of 64 keys: S^T = K . Q^T on
+// 960 patches take ~3 us of it), is shorter by that factor.  Per block of 64 keys: S^T = K . Q^T on
 // v_mfma_f32_16x16x32_f16 (lane: keys 16 j + 4 (l / 16) + i of sub-block j), in log2 units
 // (log2(e) / 8, so that every exponential is one v_exp_f32); an online softmax per query column
 // whose denominators stay per lane until the end; O^T += V^T . P^T on v_mfma_f32_16x16x16_f16 with
 // the fp16 probabilities straight from the score registers and V^T read from LDS, rescaled only
-// when some column's maximum moved.  The four parts' (max, sum, O) are combined through LDS.  Keys
-// past np are masked (their rows hold finite values; only the last block has any).  960 patches:
-// 13.4 us; with two key parts, 8 waves and unprefetched V operands 20.8.
-constexpr int VA_PARTS = 4, VA_ROW = 72, VA_TILE = 64 * VA_ROW;
-constexpr size_t VA_LDS = (size_t)VA_PARTS * 2 * 2 * VA_TILE * 2;  // [part][K, V^T][buffer]: 147,456 B
-__global__ __launch_bounds__(1024) void vit_attention_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
+// when some column's maximum moved.  The parts' (max, sum, O) are combined through LDS.  Keys past np are
+// masked (their rows hold finite values; only the last block has any).  Two parts up to ten key blocks,
+// where more waves cost more to start and to combine than they shorten (us, two / four parts: 4.7 /
+// 6.0 for 64 patches, 5.4 / 5.9 for 256, 7.9 / 8.5 for 480, 9.2 / 10.2 for 640); four above (10.5 /
+// 10.1 for 644, 10.7 / 10.2 for 768, 12.8 / 12.7 for 960).
+constexpr int VA_ROW = 72, VA_TILE = 64 * VA_ROW;
+constexpr size_t va_lds_bytes(int parts) { return (size_t)parts * 2 * 2 * VA_TILE * 2; }  // [part][K, V^T][buffer]
+template <int VA_PARTS>
+__global__ __launch_bounds__(256 * VA_PARTS) void vit_attention_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
                                                              const uint16_t* __restrict__ vt, uint16_t* __restrict__ out,
                                                              int np, int ld) {
     // V^T rows with (row / 8) odd hold their 4-key chunks pairwise swapped (chunk c at c ^ 1): the
@@ -538,10 +541,18 @@ __global__ __launch_bounds__(1024) void vit_attention_kernel(const uint16_t* __r
     }
 }
 
-hipError_t attention(const VitBuffers& b, int np, hipStream_t s) {
-    hipLaunchKernelGGL(vit_attention_kernel, dim3((np + 63) / 64, VNH), dim3(256 * VA_PARTS), VA_LDS, s, b.q, b.k, b.vt, b.attn,
-                       np, NPATCH_MAX);
+template <int PARTS>
+hipError_t attention_parts(const VitBuffers& b, int np, hipStream_t s) {
+    const hipError_t e = hipFuncSetAttribute((const void*)vit_attention_kernel<PARTS>,
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)va_lds_bytes(PARTS));
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(vit_attention_kernel<PARTS>, dim3((np + 63) / 64, VNH), dim3(256 * PARTS), va_lds_bytes(PARTS), s, b.q, b.k,
+                       b.vt, b.attn, np, NPATCH_MAX);
     return hipGetLastError();
+}
+
+hipError_t attention(const VitBuffers& b, int np, hipStream_t s) {
+    return np <= 640 ? attention_parts<2>(b, np, s) : attention_parts<4>(b, np, s);
 }
 
 template <int BN, int BM, int WN, int WM, int MODE, int S>
@@ -557,6 +568,15 @@ hipError_t gemm_deep(const VitGemmArgs& g, hipStream_t s) {
     if (g.N % 64 || g.K % 64 || g.M < 1) return hipErrorInvalidValue;
     hipLaunchKernelGGL(vit_deep_kernel<MODE>, dim3(g.N / 64, (g.M + 63) / 64), dim3(256), 0, s, g);
     return hipGetLastError();
+}
+
+// A product over a long K: 32 x 64 tiles over shared stages while every tile has a CU to itself, more
+// tiles as 64 x 64 ones with private rings.  (us, 32 x 64 / 64 x 64: fc2 17.4 / 21.5 for 64 patches,
+// 17.4 / 18.9 for 256, 17.7 / 18.5 for 512, 18.1 / 17.4 for 516, 20.0 / 18.4 for 640; a merger's first
+// product 19.2 / 23.2 for 256 patches, 19.3 / 22.7 for 512, 19.5 / 18.9 for 516, 20.7 / 20.2 for 640.)
+template <int MODE>
+hipError_t gemm_long(const VitGemmArgs& g, hipStream_t s) {
+    return g.N / 32 * ((g.M + 63) / 64) <= 256 ? gemm<32, 64, 2, 2, MODE, 4>(g, s) : gemm_deep<MODE>(g, s);
 }
 
 template <int N>
@@ -580,7 +600,7 @@ hipError_t merger(const VitMerger& mg, const uint16_t* xn, int nvis, uint16_t* h
     g.M = nvis;
     g.N = MH;
     g.K = MH;
-    VCK((gemm_deep<VG_GELU_ERF>(g, s)));
+    VCK((gemm_long<VG_GELU_ERF>(g, s)));
     g = VitGemmArgs{};
     g.X = hbuf;
     g.W = mg.fc2w;
@@ -597,7 +617,6 @@ hipError_t merger(const VitMerger& mg, const uint16_t* xn, int nvis, uint16_t* h
 hipError_t launch_vision(const VitWeights& w, const VitBuffers& b, int gh, int gw, hipStream_t s) {
     const int np = gh * gw, nvis = np / 4;
     if (gh < 2 || gw < 2 || gh % 2 || gw % 2 || np > NPATCH_MAX) return hipErrorInvalidValue;
-    VCK(hipFuncSetAttribute((const void*)vit_attention_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)VA_LDS));
     hipLaunchKernelGGL(vit_patchify_kernel, dim3(np), dim3(256), 0, s, b.rgb, b.patches, gh, gw);
     VCK(hipGetLastError());
     VitGemmArgs g{};
@@ -626,9 +645,13 @@ hipError_t launch_vision(const VitWeights& w, const VitBuffers& b, int gh, int g
         g.M = np;
         g.N = VQKV;
         g.K = VH;
-        // (a head's 64 outputs x 128 tokens: 15.7 us for 960 patches; x 64 tokens 18.6, x 192 15.6,
-        // x 256 19.3)
-        VCK((gemm<64, 128, 1, 4, VG_QKV, 3>(g, s)));
+        // A head's 64 outputs x 64 tokens while these tiles all run at once, two a CU (640 patches), x
+        // 128 above (us, x 64 / x 128: 8.7 / 12.0 for 256 patches, 11.3 / 12.2 for 480, 11.7 / 12.2 for
+        // 640, 15.6 / 13.0 for 644, 17.0 / 14.8 for 960; x 192 as x 128 there, x 256 a fifth slower).
+        if (VQKV / 64 * ((np + 63) / 64) <= 512)
+            VCK((gemm<64, 64, 1, 4, VG_QKV, 4>(g, s)));
+        else
+            VCK((gemm<64, 128, 1, 4, VG_QKV, 3>(g, s)));
         VCK(attention(b, np, s));
         g = VitGemmArgs{};
         g.X = b.attn;
@@ -658,7 +681,7 @@ hipError_t launch_vision(const VitWeights& w, const VitBuffers& b, int gh, int g
         g.M = np;
         g.N = VH;
         g.K = VFF;
-        VCK((gemm_deep<VG_F32_ADD>(g, s)));
+        VCK((gemm_long<VG_F32_ADD>(g, s)));
         if (l == 5 || l == 11 || l == 17) {
             // DeepStack merger: LayerNorm over each 2 x 2 block's 4096 values (Engine.swift:420-447).
             VCK(layernorm<MH>(b.x, w.mg[ds].nw, w.mg[ds].nb, b.xn, nvis, s));

@@ -1,6 +1,8 @@
 """GPU parity of the vision tower at patch counts where its work splits have remainders: fewer
-patches than a tile, one more than a 64-patch block, and key blocks that leave parts of the
-attention with fewer blocks than the others or none (1, 2, 3 and 5 blocks over four parts)."""
+patches than a tile, one more than a 64-patch block, key blocks that leave parts of the attention
+with fewer blocks than the others or none, and 516 patches, the first count past the small tiles of
+fc2 and the mergers' first product.  (QKV and the attention change their form past 640 patches; the
+stored frame of 960 in test_gpu_vision runs the larger one.)"""
 import numpy as np
 import pytest
 
@@ -16,7 +18,7 @@ def vimg():
     return synth.build_model_image(WeightFormat.Q4, n_layers=1, tag="q4-vision", vision=True)
 
 
-@pytest.mark.parametrize("gh,gw", [(2, 2), (2, 34), (10, 14), (10, 26)])
+@pytest.mark.parametrize("gh,gw", [(2, 2), (2, 34), (10, 14), (10, 26), (2, 258)])
 def test_tower_matches_oracle_at_remainders(oracle_mod, vimg, gh, gw):
     rgb = synth.random_rgb(gh, gw, "edges", 100 * gh + gw)
     ref_p, ref_ds = oracle_mod.vision(vimg, rgb)

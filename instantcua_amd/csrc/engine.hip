@@ -153,6 +153,18 @@ static void return_sync_area(int dev, void* p) {
     g_sync_pool.emplace_back(dev, p);
 }
 
+// Calls return with their stream idle (icua.h), whichever way they leave: until then copies from or to
+// the caller's memory may be in flight.  done(): the call has waited itself.
+struct IdleOnReturn {
+    hipStream_t stream;
+    bool waited = false;
+    explicit IdleOnReturn(hipStream_t s) : stream(s) {}
+    ~IdleOnReturn() {
+        if (!waited) (void)hipStreamSynchronize(stream);
+    }
+    void done() { waited = true; }
+};
+
 struct icua_engine {
     int fmt = 0, layers = 0, maxctx = 0, maxpass = 0, maxsteps = 0;
     uint32_t flags = 0;
@@ -507,7 +519,9 @@ struct icua_engine {
         if (write_state(s)) return -1;
         if (init_persistent()) return -1;
         if (init_vision(img, len, tab)) return -1;
-        return prepare_mrope(-1, 1, 1);
+        if (prepare_mrope(-1, 1, 1)) return -1;
+        HIPCK(hipStreamSynchronize(stream));
+        return 0;
     }
 
     // Vision tensors (ModelFile.swift:64-87, Convert.swift:97-152): copied as they are into one
@@ -681,11 +695,13 @@ struct icua_engine {
         vb.pooler = pooler;
         for (int i = 0; i < 3; ++i) vb.ds[i] = ds[i];
         if (prepare_vision_grid(gh, gw)) return -1;
+        IdleOnReturn idle(stream);
         HIPCK(hipMemcpyAsync((void*)vb.rgb, rgb, (size_t)width * height * 3, hipMemcpyHostToDevice, stream));
         HIPCK(hipEventRecord(ev0, stream));
         HIPCK(launch_vision(vw, vb, gh, gw, stream));
         HIPCK(hipEventRecord(ev1, stream));
         HIPCK(hipEventSynchronize(ev1));
+        idle.done();
         float t = 0;
         HIPCK(hipEventElapsedTime(&t, ev0, ev1));
         if (ms) *ms = t;
@@ -942,6 +958,7 @@ struct icua_engine {
         if (vis_offset >= n) return fail("vis_offset beyond the prompt");
         if (vis_offset >= 0 && n_vis <= 0) return fail("visual rows requested but no visual embeddings set");
         kv_written_from(start_pos);
+        IdleOnReturn idle(stream);
         HIPCK(hipMemcpyAsync(prompt, tokens, sizeof(int32_t) * n, hipMemcpyHostToDevice, stream));
         State s{};
         s.pos = start_pos;
@@ -966,6 +983,7 @@ struct icua_engine {
         }
         HIPCK(hipEventRecord(ev1, stream));
         HIPCK(hipEventSynchronize(ev1));
+        idle.done();
         float ms = 0;
         HIPCK(hipEventElapsedTime(&ms, ev0, ev1));
         timing.prefill_ms = ms;
@@ -998,6 +1016,7 @@ struct icua_engine {
 
     int decode_steps(int k, double* ms_out) {
         if (k < 0) return fail("negative step count");
+        IdleOnReturn idle(stream);
         bool persistent = use_persistent();
         State s;
         if (persistent) {  // single-row passes, or a pending forced pair (run as two rows)
@@ -1042,6 +1061,7 @@ struct icua_engine {
             HIPCK(hipEventRecord(ev1, stream));
         }
         HIPCK(hipEventSynchronize(ev1));
+        idle.done();
         float ms = 0;
         HIPCK(hipEventElapsedTime(&ms, ev0, ev1));
         if (ms_out) *ms_out = ms;
@@ -1293,6 +1313,7 @@ int icua_verify(icua_engine* e, const int32_t* draft, int m, int32_t* out_argmax
     if (s.pos + m > e->maxctx) return fail("verify exceeds max context");
     for (int i = 0; i < m; ++i)
         if (draft[i] < 0 || draft[i] >= VOCAB) return fail("token id out of range");
+    IdleOnReturn idle(e->stream);
     HIPCK(hipMemcpyAsync(e->prompt, draft, sizeof(int32_t) * m, hipMemcpyHostToDevice, e->stream));
     State v = s;
     v.n = m;
@@ -1319,6 +1340,7 @@ int icua_verify(icua_engine* e, const int32_t* draft, int m, int32_t* out_argmax
     if (out_logits)
         HIPCK(hipMemcpyAsync(out_logits, e->logits, sizeof(float) * (size_t)m * VOCAB, hipMemcpyDeviceToHost, e->stream));
     HIPCK(hipStreamSynchronize(e->stream));
+    idle.done();
     e->last_logits_rows = m;
     return 0;
 }
@@ -1339,6 +1361,7 @@ int icua_set_position(icua_engine* e, int pos, int32_t next_token, int step, int
     s.vis_offset = -1;
     s.logits_rows = 0;
     s.flags = (e->flags & ICUA_FLAG_GRAMMAR_PAIRS) ? STATE_FLAG_GRAMMAR : 0;
+    IdleOnReturn idle(e->stream);
     if (e->write_state(s)) return -1;
     HIPCK(hipMemcpy(e->prompt, &next_token, sizeof(int32_t), hipMemcpyHostToDevice));
     EmbedArgs ea{};
@@ -1352,6 +1375,7 @@ int icua_set_position(icua_engine* e, int pos, int32_t next_token, int step, int
     ea.n = 1;
     HIPCK(launch_embed(ea, e->stream));
     HIPCK(hipStreamSynchronize(e->stream));
+    idle.done();
     return 0;
 }
 
@@ -1396,12 +1420,16 @@ int icua_layer_step(icua_engine* e, int layer, const float* x_in, int n, int pos
     v.n = n;
     v.done = 0;
     v.vis_offset = -1;
+    IdleOnReturn idle(e->stream);
     if (e->write_state(v)) return -1;
     HIPCK(hipMemcpy(e->x, x_in, sizeof(float) * (size_t)n * H, hipMemcpyHostToDevice));
     if (e->enqueue_layer(layer, n == 1 ? 1 : MAXM, 0, n)) return -1;
     HIPCK(hipStreamSynchronize(e->stream));
     HIPCK(hipMemcpy(x_out, e->x, sizeof(float) * (size_t)n * H, hipMemcpyDeviceToHost));
-    return e->write_state(s);
+    if (e->write_state(s)) return -1;
+    HIPCK(hipStreamSynchronize(e->stream));
+    idle.done();
+    return 0;
 }
 
 static int kv_copy(icua_engine* e, int layer, int kind, int slot0, int nslots, void* host, bool to_dev) {

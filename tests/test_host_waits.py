@@ -1,0 +1,74 @@
+"""CPU tests of what the engine's calls wait for, against a HIP runtime of host memory
+(fake_hip.c): calls are synchronous (icua.h), so none returns with work or copies of the caller's
+memory pending on its stream, and an error return in the middle of a pass does not either."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+
+def _run(fake, body):
+    code = f"""
+import ctypes as C, sys
+sys.path.insert(0, {os.path.dirname(HERE)!r})
+import numpy as np
+from instantcua_amd import synth
+from instantcua_amd.engine import Engine, EngineError
+from instantcua_amd.modelfile import WeightFormat
+fake = C.CDLL({fake!r})
+e = Engine(flags=0, image=synth.build_model_image(WeightFormat.Q4, 1, tag="waits"), max_context=64, max_steps=4)
+assert fake.fake_busy() == 0, "create"
+toks = np.arange(20, dtype=np.int32)
+calls = {{
+    "prefill": lambda: e.prefill(toks, max_new=2, write_logits=True),
+    "passes": lambda: e.prefill(toks[:5], max_new=2),
+    "verify": lambda: e.verify(toks[:3]),
+    "verify_logits": lambda: e.verify(toks[:3], want_logits=True),
+    "set_position": lambda: e.set_position(3, 7),
+    "decode": lambda: e.decode_steps(2),
+    "layer_step": lambda: e.layer_step(0, np.zeros((2, 2048), np.float32), 3),
+}}
+{body}
+print("done")
+"""
+    preload = ":".join(filter(None, [fake, os.environ.get("LD_PRELOAD")]))
+    r = subprocess.run([sys.executable, "-c", code], env={**os.environ, "LD_PRELOAD": preload}, capture_output=True,
+                       text=True, timeout=300)
+    assert r.returncode == 0 and r.stdout.strip().endswith("done"), r.stdout[-2000:] + r.stderr[-2000:]
+
+
+@pytest.fixture(scope="module")
+def fake(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("hip") / "libfakehip.so")
+    subprocess.run(["gcc", "-O1", "-shared", "-fPIC", "-o", so, os.path.join(HERE, "fake_hip.c")], check=True)
+    return so
+
+
+def test_calls_return_with_nothing_pending(fake):
+    _run(fake, """
+for name, call in calls.items():
+    call()
+    assert fake.fake_busy() == 0, name
+""")
+
+
+def test_error_returns_leave_nothing_pending(fake):
+    """Every kernel launch of a call fails in turn."""
+    _run(fake, """
+for name, call in calls.items():
+    call()
+    fake.fake_arm(0)
+    call()
+    n = fake.fake_launches()  # (a decode has none: it replays the graph of its first call)
+    for k in range(1, n + 1):
+        fake.fake_arm(k)
+        try:
+            call()
+            raise SystemExit(f"{name}: launch {k} of {n} failed unseen")
+        except EngineError:
+            pass
+        assert fake.fake_busy() == 0, f"{name}: launch {k} of {n}"
+""")

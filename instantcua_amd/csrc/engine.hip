@@ -1439,13 +1439,21 @@ static int kv_copy(icua_engine* e, int layer, int kind, int slot0, int nslots, v
     if (slot0 < 0 || nslots < 0 || slot0 + nslots > e->maxctx) return fail("slots out of range");
     if (to_dev && nslots > 0) e->kv_written_from(slot0);
     if (nslots == 0) return 0;
-    // The KV groups' slot ranges in one strided copy.
-    uint16_t* dev = e->kv_ptr(layer, kind) + (size_t)slot0 * HD;
+    // The KV groups' slot ranges in one strided copy, or between 16 and 128 KiB a group one by one (us
+    // to write, strided / one by one: 64 slots 79 / 97, 96 80 / 75, 256 90 / 82, 448 95 / 95, 640 103 /
+    // 108, 4096 239 / 330; to read, 64 slots 67 / 101, from 96 on the same).
+    uint8_t* dev = (uint8_t*)(e->kv_ptr(layer, kind) + (size_t)slot0 * HD);
+    uint8_t* hp = (uint8_t*)host;
     const size_t row = (size_t)nslots * HD * 2, pitch = (size_t)e->maxctx * HD * 2;
-    if (to_dev)
-        HIPCK(hipMemcpy2D(dev, pitch, host, row, row, NKV, hipMemcpyHostToDevice));
-    else
-        HIPCK(hipMemcpy2D(host, row, dev, pitch, row, NKV, hipMemcpyDeviceToHost));
+    const int each = row > 16384 && row < 131072 ? 1 : NKV;  // groups of a copy
+    for (int g = 0; g < NKV; g += each) {
+        if (to_dev)
+            HIPCK(each == 1 ? hipMemcpy(dev + g * pitch, hp + g * row, row, hipMemcpyHostToDevice)
+                            : hipMemcpy2D(dev, pitch, hp, row, row, NKV, hipMemcpyHostToDevice));
+        else
+            HIPCK(each == 1 ? hipMemcpy(hp + g * row, dev + g * pitch, row, hipMemcpyDeviceToHost)
+                            : hipMemcpy2D(hp, row, dev, pitch, row, NKV, hipMemcpyDeviceToHost));
+    }
     return 0;
 }
 

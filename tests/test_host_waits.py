@@ -1,6 +1,7 @@
-"""CPU tests of what the engine's calls wait for, against a HIP runtime of host memory
-(fake_hip.c): calls are synchronous (icua.h), so none returns with work or copies of the caller's
-memory pending on its stream, and an error return in the middle of a pass does not either."""
+"""CPU tests of the engine's host code, against a HIP runtime of host memory (fake_hip.c).  Calls are
+synchronous (icua.h): none returns with work or copies of the caller's memory pending on its stream,
+and an error return in the middle of a pass does not either.  K/V ranges land where they belong in
+every form of the copy."""
 import os
 import subprocess
 import sys
@@ -19,7 +20,7 @@ from instantcua_amd import synth
 from instantcua_amd.engine import Engine, EngineError
 from instantcua_amd.modelfile import WeightFormat
 fake = C.CDLL({fake!r})
-e = Engine(flags=0, image=synth.build_model_image(WeightFormat.Q4, 1, tag="waits"), max_context=64, max_steps=4)
+e = Engine(flags=0, image=synth.build_model_image(WeightFormat.Q4, 1, tag="waits"), max_context=600, max_steps=4)
 assert fake.fake_busy() == 0, "create"
 toks = np.arange(20, dtype=np.int32)
 calls = {{
@@ -71,4 +72,20 @@ for name, call in calls.items():
         except EngineError:
             pass
         assert fake.fake_busy() == 0, f"{name}: launch {k} of {n}"
+""")
+
+
+def test_kv_ranges_round_trip(fake):
+    """Sizes on either side of the changes between one strided copy and a copy a group."""
+    _run(fake, """
+rng = np.random.default_rng(0)
+for kind in (0, 1):
+    full = rng.integers(0, 1 << 16, (8, 600, 128)).astype(np.uint16).view(np.float16)
+    e.write_kv(0, kind, 0, full)
+    for slot0, n in ((0, 600), (3, 1), (5, 64), (5, 65), (7, 511), (7, 512), (599, 1)):
+        new = rng.integers(0, 1 << 16, (8, n, 128)).astype(np.uint16).view(np.float16)
+        full[:, slot0:slot0 + n] = new
+        e.write_kv(0, kind, slot0, new)
+        assert np.array_equal(e.read_kv(0, kind, slot0, n).view(np.uint16), new.view(np.uint16)), n
+        assert np.array_equal(e.read_kv(0, kind, 0, 600).view(np.uint16), full.view(np.uint16)), n
 """)

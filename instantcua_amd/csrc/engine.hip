@@ -206,7 +206,9 @@ struct icua_engine {
     // Matrix-core prefill buffers for chunks of up to pf_cap rows (allocated on first use).
     int pf_cap = 0;
     float *px = nullptr, *pqkv = nullptr, *patt = nullptr, *ph = nullptr, *pts = nullptr;
-    float *ppart = nullptr, *ppml = nullptr;  // K-split GEMM and key-split attention partials
+    // K-split GEMM and key-split attention partials: their sizes do not depend on the prompt, so they are
+    // allocated once.
+    float *ppart = nullptr, *ppml = nullptr;
     uint16_t *pxa = nullptr, *pxb = nullptr, *pqh = nullptr, *pql = nullptr;
     // Vision tower, when the image holds it: weights, work buffers (one allocation, on first
     // use), the host copy of the position table, the prepared grid and the frame hash.
@@ -780,15 +782,17 @@ struct icua_engine {
     }
 
     void free_pf() {
-        void* bufs[] = {px, pqkv, patt, ph, pts, pxa, pxb, pqh, pql, ppart, ppml};
+        void* bufs[] = {px, pqkv, patt, ph, pts, pxa, pxb, pqh, pql};
         for (void* b : bufs)
             if (b) (void)hipFree(b);
-        px = pqkv = patt = ph = pts = ppart = ppml = nullptr;
+        px = pqkv = patt = ph = pts = nullptr;
         pxa = pxb = pqh = pql = nullptr;
         pf_cap = 0;
     }
 
     int ensure_pf(int rows) {
+        if (!ppart) HIPCK(hipMalloc(&ppart, sizeof(float) * PF_PART_FLOATS));
+        if (!ppml) HIPCK(hipMalloc(&ppml, sizeof(float) * PF_PART_ML_FLOATS));
         const int cap = (rows + 127) / 128 * 128;
         if (cap <= pf_cap) return 0;
         HIPCK(hipStreamSynchronize(stream));
@@ -799,8 +803,6 @@ struct icua_engine {
         HIPCK(hipMalloc(&ph, sizeof(float) * cap * FF));
         HIPCK(hipMalloc(&pxa, sizeof(uint16_t) * 2 * (size_t)cap * FF));
         HIPCK(hipMalloc(&pxb, sizeof(uint16_t) * (size_t)cap / 16 * (FF / 2048) * 2 * 512));
-        HIPCK(hipMalloc(&ppart, sizeof(float) * PF_PART_FLOATS));
-        HIPCK(hipMalloc(&ppml, sizeof(float) * PF_PART_ML_FLOATS));
         HIPCK(hipMalloc(&pts, sizeof(float) * (size_t)cap));
         HIPCK(hipMalloc(&pqh, sizeof(uint16_t) * (size_t)cap * NH * HD));
         HIPCK(hipMalloc(&pql, sizeof(uint16_t) * (size_t)cap * NH * HD));
@@ -1117,7 +1119,7 @@ void icua_engine_destroy(icua_engine* e) {
         if (g) (void)hipGraphExecDestroy(g);
     void* bufs[] = {e->d_weights, e->x, e->qkv, e->attn, e->h, e->kv, e->rope, e->part, e->counters, e->kpart, e->kcnt, e->apre, e->fxpre, e->pval,
                     e->pidx, e->logits, e->out_tokens, e->prompt, e->argmax_rows, e->st, e->pooler,
-                    e->ds[0], e->ds[1], e->ds[2], e->d_vision, e->vbuf};
+                    e->ds[0], e->ds[1], e->ds[2], e->d_vision, e->vbuf, e->ppart, e->ppml};
     if (e->psync) return_sync_area(e->psync_dev, e->psync);
     e->free_pf();
     for (void* b : bufs)

@@ -8,11 +8,15 @@
 
 enum { OK = 0, FAILED = 719 /* hipErrorLaunchFailure */, STREAMS = 64 };
 static int busy[STREAMS], nstream = 1, launches, fail_at, capturing;
+static int live; /* allocations not freed */
+static size_t big; /* bytes of allocations of more than 32 MiB since fake_arm() */
 static uintptr_t last_error;
 
 static int idx(void* s) { return (int)(uintptr_t)s; } /* stream 0: the null stream */
 
-void fake_arm(int k) { launches = 0, fail_at = k; }
+void fake_arm(int k) { launches = 0, fail_at = k, big = 0; }
+int fake_live(void) { return live; }
+size_t fake_big(void) { return big; }
 int fake_launches(void) { return launches; }
 int fake_busy(void) { /* operations not waited for */
     int n = 0;
@@ -20,9 +24,9 @@ int fake_busy(void) { /* operations not waited for */
     return n;
 }
 
-int hipMalloc(void** p, size_t n) { return *p = calloc(1, n ? n : 1), OK; }
+int hipMalloc(void** p, size_t n) { return ++live, big += n >= 32u << 20 ? n : 0, *p = calloc(1, n ? n : 1), OK; }
 int hipExtMallocWithFlags(void** p, size_t n, unsigned f) { return (void)f, hipMalloc(p, n); }
-int hipFree(void* p) { return free(p), OK; }
+int hipFree(void* p) { return live -= p != NULL, free(p), OK; }
 int hipMemcpy(void* d, const void* s, size_t n, int k) { return (void)k, memmove(d, s, n), OK; }
 int hipMemcpyAsync(void* d, const void* s, size_t n, int k, void* st) { return (void)k, memmove(d, s, n), ++busy[idx(st)], OK; }
 int hipMemcpyWithStream(void* d, const void* s, size_t n, int k, void* st) { return (void)k, memmove(d, s, n), busy[idx(st)] = 0, OK; }

@@ -89,3 +89,20 @@ for kind in (0, 1):
         assert np.array_equal(e.read_kv(0, kind, slot0, n).view(np.uint16), new.view(np.uint16)), n
         assert np.array_equal(e.read_kv(0, kind, 0, 600).view(np.uint16), full.view(np.uint16)), n
 """)
+
+
+def test_prefill_buffers(fake):
+    """The partials' buffer is allocated once, whatever prompts follow, and closing frees everything.
+    (Of the others none reaches 32 MiB at these sizes.)"""
+    _run(fake, """
+fake.fake_big.restype = C.c_size_t
+fake.fake_arm(0)
+e.prefill(toks[:9], max_new=2)
+assert fake.fake_big() == 4 * 256 * 128 * 256, fake.fake_big()
+fake.fake_arm(0)
+for n in (20, 200, 400, 590):
+    e.prefill(np.arange(n, dtype=np.int32), max_new=2)
+assert fake.fake_big() == 0, fake.fake_big()
+e.close()
+assert fake.fake_live() == 0, fake.fake_live()
+""")

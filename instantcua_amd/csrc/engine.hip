@@ -806,9 +806,10 @@ struct icua_engine {
         HIPCK(hipMalloc(&pts, sizeof(float) * (size_t)cap));
         HIPCK(hipMalloc(&pqh, sizeof(uint16_t) * (size_t)cap * NH * HD));
         HIPCK(hipMalloc(&pql, sizeof(uint16_t) * (size_t)cap * NH * HD));
-        // Rows beyond a chunk's M are read (never stored) by the attention kernel: keep them finite.
-        HIPCK(hipMemset(pqh, 0, sizeof(uint16_t) * (size_t)cap * NH * HD));
-        HIPCK(hipMemset(pql, 0, sizeof(uint16_t) * (size_t)cap * NH * HD));
+        // Rows beyond a chunk's M are read (never stored) by the attention kernel: keep them finite.  On
+        // the engine's stream, which does not wait for the null stream's (asynchronous) hipMemset.
+        HIPCK(hipMemsetAsync(pqh, 0, sizeof(uint16_t) * (size_t)cap * NH * HD, stream));
+        HIPCK(hipMemsetAsync(pql, 0, sizeof(uint16_t) * (size_t)cap * NH * HD, stream));
         pf_cap = cap;
         return 0;
     }

@@ -8,13 +8,15 @@
 
 enum { OK = 0, FAILED = 719 /* hipErrorLaunchFailure */, STREAMS = 64 };
 static int busy[STREAMS], nstream = 1, launches, fail_at, capturing;
+static int overlaps; /* launches on other streams while the null stream has work, since fake_arm() */
 static int live; /* allocations not freed */
 static size_t big; /* bytes of allocations of more than 32 MiB since fake_arm() */
 static uintptr_t last_error;
 
 static int idx(void* s) { return (int)(uintptr_t)s; } /* stream 0: the null stream */
 
-void fake_arm(int k) { launches = 0, fail_at = k, big = 0; }
+void fake_arm(int k) { launches = 0, fail_at = k, big = 0, overlaps = 0; }
+int fake_overlaps(void) { return overlaps; }
 int fake_live(void) { return live; }
 size_t fake_big(void) { return big; }
 int fake_launches(void) { return launches; }
@@ -27,15 +29,15 @@ int fake_busy(void) { /* operations not waited for */
 int hipMalloc(void** p, size_t n) { return ++live, big += n >= 32u << 20 ? n : 0, *p = calloc(1, n ? n : 1), OK; }
 int hipExtMallocWithFlags(void** p, size_t n, unsigned f) { return (void)f, hipMalloc(p, n); }
 int hipFree(void* p) { return live -= p != NULL, free(p), OK; }
-int hipMemcpy(void* d, const void* s, size_t n, int k) { return (void)k, memmove(d, s, n), OK; }
+int hipMemcpy(void* d, const void* s, size_t n, int k) { return (void)k, memmove(d, s, n), busy[0] = 0, OK; }
 int hipMemcpyAsync(void* d, const void* s, size_t n, int k, void* st) { return (void)k, memmove(d, s, n), ++busy[idx(st)], OK; }
 int hipMemcpyWithStream(void* d, const void* s, size_t n, int k, void* st) { return (void)k, memmove(d, s, n), busy[idx(st)] = 0, OK; }
 int hipMemcpy2D(void* d, size_t dp, const void* s, size_t sp, size_t w, size_t h, int k) {
     (void)k;
     for (size_t i = 0; i < h; ++i) memmove((char*)d + i * dp, (const char*)s + i * sp, w);
-    return OK;
+    return busy[0] = 0, OK;
 }
-int hipMemset(void* d, int v, size_t n) { return memset(d, v, n), OK; }
+int hipMemset(void* d, int v, size_t n) { return memset(d, v, n), ++busy[0], OK; } /* returns before it is done */
 int hipMemsetAsync(void* d, int v, size_t n, void* st) { return memset(d, v, n), ++busy[idx(st)], OK; }
 int hipStreamCreateWithFlags(void** s, unsigned f) { return (void)f, *s = (void*)(uintptr_t)nstream++, OK; }
 int hipStreamDestroy(void* s) { return (void)s, OK; }
@@ -61,6 +63,7 @@ int hipGraphLaunch(void* x, void* s) { return (void)x, ++busy[idx(s)], OK; }
 typedef struct { unsigned x, y, z; } dim3_;
 int hipLaunchKernel(const void* f, dim3_ g, dim3_ b, void** a, size_t l, void* st) {
     (void)f, (void)g, (void)b, (void)a, (void)l;
+    overlaps += st && busy[0];
     if (++launches == fail_at) return last_error = FAILED;
     return busy[idx(st)] += !capturing, OK;
 }

@@ -91,6 +91,19 @@ for kind in (0, 1):
 """)
 
 
+def test_null_stream_work_is_waited_for(fake):
+    """The engine's stream does not wait for the null stream: nothing starts on it while a clear of
+    new buffers may be running there."""
+    _run(fake, """
+fake.fake_arm(0)
+for name, call in calls.items():
+    call()
+    assert fake.fake_overlaps() == 0, name
+e.prefill(np.arange(300, dtype=np.int32), max_new=2)
+assert fake.fake_overlaps() == 0, "longer prefill"
+""")
+
+
 def test_prefill_buffers(fake):
     """The partials' buffer is allocated once, whatever prompts follow, and closing frees everything.
     (Of the others none reaches 32 MiB at these sizes.)"""

@@ -10,15 +10,17 @@ enum { OK = 0, FAILED = 719 /* hipErrorLaunchFailure */, STREAMS = 64 };
 static int busy[STREAMS], nstream = 1, launches, fail_at, capturing;
 static int overlaps; /* launches on other streams while the null stream has work, since fake_arm() */
 static int live; /* allocations not freed */
-static size_t big; /* bytes of allocations of more than 32 MiB since fake_arm() */
+static size_t watched; /* allocations of exactly this size are counted */
+static int seen;
 static uintptr_t last_error;
 
 static int idx(void* s) { return (int)(uintptr_t)s; } /* stream 0: the null stream */
 
-void fake_arm(int k) { launches = 0, fail_at = k, big = 0, overlaps = 0; }
+void fake_arm(int k) { launches = 0, fail_at = k, overlaps = 0; }
 int fake_overlaps(void) { return overlaps; }
 int fake_live(void) { return live; }
-size_t fake_big(void) { return big; }
+void fake_watch(size_t n) { watched = n, seen = 0; }
+int fake_seen(void) { return seen; }
 int fake_launches(void) { return launches; }
 int fake_busy(void) { /* operations not waited for */
     int n = 0;
@@ -26,7 +28,7 @@ int fake_busy(void) { /* operations not waited for */
     return n;
 }
 
-int hipMalloc(void** p, size_t n) { return ++live, big += n >= 32u << 20 ? n : 0, *p = calloc(1, n ? n : 1), OK; }
+int hipMalloc(void** p, size_t n) { return ++live, seen += n == watched, *p = calloc(1, n ? n : 1), OK; }
 int hipExtMallocWithFlags(void** p, size_t n, unsigned f) { return (void)f, hipMalloc(p, n); }
 int hipFree(void* p) { return live -= p != NULL, free(p), OK; }
 int hipMemcpy(void* d, const void* s, size_t n, int k) { return (void)k, memmove(d, s, n), busy[0] = 0, OK; }

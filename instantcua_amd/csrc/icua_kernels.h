@@ -148,17 +148,19 @@ struct PfGemmArgs {
     int splits;             // pf_gemm_splits(): > 1 stores K-split partials [splits][M][N] to part
     float* part;
 };
-// Chunks of up to this many rows take the K-split GEMM, larger ones the 128-token tiles, by the
-// weights and the operand parts (a chunk has at most 4096).  The lines lie where the two meet (4
-// layers and the head, split / 128-token tiles, ms): hi + lo q4 1.30 / 1.31 at 1000 rows, 2.09 / 2.27
-// at 1536, 2.53 / 2.37 at 2048 (q8 2.28 / 2.47 and 2.80 / 2.56).  fp16 operands alone q8 1.67 / 1.72 at
-// 2048, 2.58 / 2.49 at 3000; q4 1.49 / 1.61 and 2.28 / 2.42, 2.89 / 2.95 at 4096.  f16 weights are
-// ahead at every size (4096 rows: 4.95 / 5.28, fp16 operands 3.22 / 3.29).
-inline int pf_split_rows(int fmt, int parts) {
-    if (fmt == FMT_F16 || (fmt == FMT_Q4 && parts == 1)) return 4096;
-    return parts == 2 ? 1536 : 2048;
+// Whether a chunk of M rows takes the K-split GEMM or the 128-token tiles, by the weights and the
+// operand parts (a chunk has at most 4096).  The lines lie where the two meet (4 layers and the head,
+// split / 128-token tiles, ms): hi + lo q4 1.30 / 1.31 at 1000 rows, 2.09 / 2.27 at 1536, 2.53 / 2.37 at
+// 2048 (q8 2.28 / 2.47 and 2.80 / 2.56).  fp16 operands alone q8 1.67 / 1.72 at 2048, 2.58 / 2.49 at
+// 3000; q4 1.49 / 1.61 and 2.28 / 2.42, 2.89 / 2.95 at 4096.  f16 weights are ahead at every size with
+// fp16 operands alone (4096 rows 3.22 / 3.29), and with hi + lo (4096 rows 4.95 / 5.28) but for 2049 -
+// 2304 rows, where the 264-288 tiles of O and down leave a second wave nearly empty (2100 rows 3.33 /
+// 3.18, 2300 rows 3.36 / 3.25; 2400 rows 3.38 / 3.43).
+inline bool pf_use_split(int fmt, int parts, int M) {
+    if (fmt == FMT_F16) return parts == 1 || M <= 2048 || M > 2304;
+    if (fmt == FMT_Q4 && parts == 1) return true;
+    return M <= (parts == 2 ? 1536 : 2048);
 }
-inline bool pf_use_split(int fmt, int parts, int M) { return M <= pf_split_rows(fmt, parts); }
 int pf_gemm_splits(int fmt, int parts, int K, int N, int M);
 // Partials of a GEMM (at most 256 tiles of 128 x 256) or an attention (256 / 8 query
 // blocks and splits of 64 rows), floats.

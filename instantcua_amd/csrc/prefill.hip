@@ -345,24 +345,24 @@ __device__ __forceinline__ void pf_store(const PfGemmArgs& a, int t, int row, fl
 // blocks per wave, RB = 8 or 16 row blocks); wave w owns token blocks 4 TB tm + TB (w % 4) ..
 // against row blocks RB / 2 (w / 4) onwards (RB / 2 row blocks), two waves per SIMD, and takes
 // its row blocks in halves of four per group.  Each 128-K step, the weight chunks of the RB row
-// blocks (q4 one 1 KiB chunk, q8 two) become fp16 B operands in LDS once
+// blocks (q4 one 1 KiB chunk, q8 two, f16 four) become fp16 B operands in LDS once
 // (double-buffered, 64 or 128 KiB) and are shared by the waves; the waves' activation operands
 // stream from global memory straight into registers two 64-K groups ahead.  The launch takes
 // the largest tile (most products per operand byte) whose count still fills the CUs evenly.
 template <int FMT, int K, int EPI, int PG_RB, int TB, int HL>
 __global__ __launch_bounds__(512) void pf_gemm_kernel(PfGemmArgs a) {
     static_assert((PG_RB == 8 || PG_RB == 16) && (TB == 1 || TB == 2), "tile shape");
-    static_assert(FMT == FMT_Q8 || (FMT == FMT_Q4 && HL == 2), "the other prompts take the K-split GEMM");
+    static_assert(FMT == FMT_Q8 || HL == 2, "q4 and f16 with fp16 operands alone take the K-split GEMM");
     constexpr int NHF = PG_RB / 8;         // halves of four row blocks per wave
     constexpr int TR = 16 * PG_RB;         // rows of a tile
     constexpr int NG = K / 64, NKS = K / 32, NC = K / 128;
-    constexpr int CPS = FMT == FMT_Q4 ? 1 : 2;  // 1 KiB chunks per 128-K step
+    constexpr int CPS = FMT == FMT_Q4 ? 1 : FMT == FMT_Q8 ? 2 : 4;  // 1 KiB chunks per 128-K step
     constexpr int NCH = NC * CPS;                                      // chunks per row block
     // DQ: the B operands are the dequantised q8 weights s q in fp16 (the reference engine's prefill
-    // precision, taken with fp16 operands alone), so the products accumulate straight into the
-    // outputs; otherwise codes are exact fp16 integers and each group's sums take their scale in an
-    // epilogue.
-    constexpr bool DQ = HL == 1;
+    // precision, taken with fp16 operands alone) or the f16 weights themselves, so the products
+    // accumulate straight into the outputs; otherwise codes are exact fp16 integers and each group's
+    // sums take their scale in an epilogue.
+    constexpr bool DQ = HL == 1 || FMT == FMT_F16;
     const int TN = a.N / (16 * PG_RB), TM = a.Mpad / (64 * TB), T = TM * TN;
     const int per = (T + 7) / 8;
     const int tile = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);
@@ -419,7 +419,7 @@ __global__ __launch_bounds__(512) void pf_gemm_kernel(PfGemmArgs a) {
 #pragma unroll
             for (int j = 0; j < CPS; ++j) Wn[hb][j] = *(const uint4*)(wsrc + hb * WSRC2 + (size_t)(c * CPS + j) * 1024);
         if (vload) Vn = vsrc[(size_t)c * vstride];
-        if constexpr (DQ) {
+        if constexpr (DQ && FMT != FMT_F16) {  // f16 weights have no scales
 #pragma unroll
             for (int hb = 0; hb < NHF; ++hb)
 #pragma unroll
@@ -431,7 +431,10 @@ __global__ __launch_bounds__(512) void pf_gemm_kernel(PfGemmArgs a) {
 #pragma unroll
         for (int hb = 0; hb < NHF; ++hb) {
             const int sr = srb + 8 * hb;
-            if constexpr (FMT == FMT_Q8) {
+            if constexpr (FMT == FMT_F16) {  // chunk j is k-step j
+#pragma unroll
+                for (int j = 0; j < 4; ++j) Bs[b][sr][j][lane] = Wn[hb][j];
+            } else if constexpr (FMT == FMT_Q8) {
                 // Bytes 0-7 of a lane of chunk j are k-step 2 j, bytes 8-15 k-step 2 j + 1.
 #pragma unroll
                 for (int j = 0; j < 2; ++j) {
@@ -1359,12 +1362,13 @@ static hipError_t pf_gemm_shape(int K, int epi, const PfGemmArgs& a, hipStream_t
 static bool even_fill(int tiles) { return tiles >= 256 && (tiles % 256 == 0 || tiles >= 1024); }
 
 // The largest tile whose count fills the CUs evenly: 128 tokens x 256 rows, 128 x 128, else
-// 64 x 128.  fp16 operands alone keep 128-row tiles: their 128-row tile needs ~110 registers and 64 KiB of LDS, so two
+// 64 x 128.  f16 weights keep 128-row tiles (their four chunks a step would not fit the registers of
+// the larger one).  fp16 operands alone keep 128-row tiles: their 128-row tile needs ~110 registers and 64 KiB of LDS, so two
 // workgroups share a CU (measured 21.55 -> 20.97 ms per 4096-row prefill against 256-row tiles).
 template <int FMT, int HL>
 static hipError_t pf_gemm_fmt(int K, int epi, const PfGemmArgs& a, hipStream_t s) {
     const int tm128 = a.Mpad / 128;
-    if constexpr (HL == 2)
+    if constexpr (HL == 2 && FMT != FMT_F16)
         if (even_fill(tm128 * (a.N / 256))) return pf_gemm_shape<FMT, 16, 2, HL>(K, epi, a, s);
     if (even_fill(tm128 * (a.N / 128))) return pf_gemm_shape<FMT, 8, 2, HL>(K, epi, a, s);
     return pf_gemm_shape<FMT, 8, 1, HL>(K, epi, a, s);
@@ -1444,7 +1448,8 @@ hipError_t launch_pf_gemm(int fmt, int K, int epi, const PfGemmArgs& a, hipStrea
     if (a.Mpad < a.M || a.Mpad % 128 || a.splits != 1) return hipErrorInvalidValue;
     if (fmt == FMT_Q8) return a.parts == 2 ? pf_gemm_fmt<FMT_Q8, 2>(K, epi, a, s) : pf_gemm_fmt<FMT_Q8, 1>(K, epi, a, s);
     if (fmt == FMT_Q4 && a.parts == 2) return pf_gemm_fmt<FMT_Q4, 2>(K, epi, a, s);
-    return hipErrorInvalidValue;  // pf_split_rows sends every other chunk the other way
+    if (fmt == FMT_F16 && a.parts == 2) return pf_gemm_fmt<FMT_F16, 2>(K, epi, a, s);
+    return hipErrorInvalidValue;  // pf_use_split sends every other chunk the other way
 }
 
 hipError_t launch_pf_qk(const PfQkArgs& a, hipStream_t s) {

@@ -69,9 +69,11 @@ def test_split_prefill_matches_passes(fmt, n, start):
 # hi + lo: the last size of four 64-token tiles (O and down change their width), of the K-split GEMM
 # and one past each.  fp16 operands: the first sizes of the 128-token tiles of the K-split GEMM (q8
 # 192, f16 320, q4 1152) and the first past it (q8 2049).  Past the K-split GEMM, where the tile of a
-# product follows its count: 2000 rows (O and down on 128 x 128) and 3000 rows (QKV on 128 x 128).
+# product follows its count: 2000 rows (O and down on 128 x 128) and 3000 rows (QKV on 128 x 128); f16
+# takes these tiles from 2049 to 2304 rows.
 @pytest.mark.parametrize("fmt,n", [("q4", 256), ("q8", 257), ("q4", 1536), ("q4", 1537), ("q8", 191), ("q8", 192),
-                                   ("f16", 320), ("q4", 1152), ("q8", 2049), ("q8", 2000), ("q8", 3000)])
+                                   ("f16", 320), ("q4", 1152), ("q8", 2049), ("q8", 2000), ("q8", 3000), ("f16", 2100),
+                                   ("f16", 2305)])
 def test_sizes_where_the_tiles_change_match_passes(fmt, n):
     check(image(fmt), synth.random_tokens(n, f"split-{n}"))
 

@@ -181,17 +181,17 @@ def test_two_chunks_match_pass_path(q4_small):
 @pytest.mark.parametrize("fmt", [WeightFormat.Q8, WeightFormat.F16], ids=["q8", "f16"])
 @pytest.mark.parametrize("n", [1024, 4096])
 def test_large_tile_prefill_matches_oracle(oracle_mod, n, fmt):
-    """Prompts long enough for the larger GEMM tiles (prefill.hip pf_gemm_fmt picks the largest
-    tile whose count fills the 256 CUs evenly), q8 and f16, against the oracle run live:
+    """Long prompts, q8 and f16, against the oracle run live:
 
-      n = 1024: q8 QKV and gate|up on 128 x 128 tiles (8 row-tiles x 32 / 96 column tiles), O and
-                down on 64 x 128; f16 the same.
-      n = 4096: q8 every GEMM on 128 x 256 tiles (32 x 16 / 8 / 48 / 8 tiles); f16 (never 256-row
-                tiles) every GEMM on 128 x 128.
+      n = 1024: every GEMM K-split, on 64 x 256 tiles.
+      n = 4096: q8 every GEMM on 128 x 256 tiles over the whole K (32 x 16 / 8 / 48 / 8 tiles;
+                prefill.hip pf_gemm_fmt picks the largest tile whose count fills the 256 CUs
+                evenly); f16 on the K-split GEMM's 64 x 256 tiles, unsplit.
 
-    Checked: first logits within 1e-4, K/V rows of the last layer at spread slots, first greedy
-    tokens; then the same prompt with fp16 operands alone (ICUA_FLAG_PREFILL_FP16, whose q8 GEMMs
-    keep 128-row tiles and take the dequantised weights as B operands) against the same oracle
+    (The other tiles over the whole K are in test_gpu_prefill_split.)  Checked: first logits within
+    1e-4, K/V rows of the last layer at spread slots, first greedy tokens; then the same prompt with
+    fp16 operands alone (ICUA_FLAG_PREFILL_FP16, which takes the dequantised weights as B operands:
+    K-split tiles of 128 tokens, for q8 at n = 4096 128 x 128 over the whole K) against the same oracle
     run: first logits within 1e-2, K/V rows within 1e-2 of their row, the first greedy token."""
     img = small_image(fmt)
     toks = synth.random_tokens(n, f"pf-large-{n}")

@@ -72,7 +72,8 @@ def test_split_prefill_matches_passes(fmt, n, start):
 # product follows its count: 2000 rows (O and down on 128 x 128) and 3000 rows (QKV on 128 x 128); f16
 # takes these tiles from 2049 to 2304 rows.
 @pytest.mark.parametrize("fmt,n", [("q4", 256), ("q8", 257), ("q4", 1536), ("q4", 1537), ("q8", 191), ("q8", 192),
-                                   ("f16", 320), ("q4", 1152), ("q8", 2049), ("q8", 2000), ("q8", 3000), ("f16", 2100),
+                                   ("f16", 320), ("q4", 1152), ("q8", 2049), ("q4", 2000), ("q8", 2000),
+                                   ("q4", 3000), ("q8", 3000), ("f16", 2100),
                                    ("f16", 2305)])
 def test_sizes_where_the_tiles_change_match_passes(fmt, n):
     check(image(fmt), synth.random_tokens(n, f"split-{n}"))
@@ -83,4 +84,12 @@ def test_split_visual_prefill_matches_passes(tail):
     """DeepStack rows are added where the down projection's partials are summed; the last layer's
     by the row that the head reads, visual or not."""
     vp = synth.visual_prompt(16 + 96 + tail, vis_offset=16, llm_h=8, llm_w=12, tag="split-vis")
+    check(image("q4"), vp.tokens, 0, vp)
+
+
+@pytest.mark.parametrize("n", [4192, 4300], ids=["last-row-visual", "text-after"])
+def test_visual_rows_in_a_second_chunk_match_passes(n):
+    """192 visual rows across the 4096-row chunks: DeepStack rows from the 97th on belong to the
+    second chunk, whose down projections leave partials."""
+    vp = synth.visual_prompt(n, vis_offset=4000, llm_h=12, llm_w=16, tag="split-vis2")
     check(image("q4"), vp.tokens, 0, vp)

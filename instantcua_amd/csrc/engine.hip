@@ -309,6 +309,7 @@ struct icua_engine {
         a.ds_row0 = row0;
         a.kpart = kpart;
         a.kcnt = kcnt;
+        a.krows = H;
         if (gemv(GEMV_DOWN, a, mt)) return -1;
         return 0;
     }
@@ -1533,10 +1534,9 @@ static int gemv_setup(int fmt, int N, int K, int m, GemvArgs& a, GemvOp& op) {
     if (standalone_buffers(b)) return -1;
     a = GemvArgs{};
     a.st = b.st;
-    if (N <= GEMV_SPLIT_ROWS) {
-        a.kpart = b.kpart;
-        a.kcnt = b.kcnt;
-    }
+    a.kpart = b.kpart;
+    a.kcnt = b.kcnt;
+    a.krows = GEMV_SPLIT_ROWS;
     a.m_fixed = m;
     a.N = N;
     op = (K == H) ? GEMV_PLAIN : GEMV_PLAIN_K6144;

@@ -618,7 +618,7 @@ static hipError_t gemv_fmt(GemvOp op, const GemvArgs& a, int mt, hipStream_t s) 
             return one ? launch_one<FMT, H, 4, 1, PRO_NORM, EPI_SWIGLU>(a, FF / 8, s)
                        : launch_one<FMT, H, 4, MAXM, PRO_NORM, EPI_SWIGLU>(a, FF / 8, s);
         case GEMV_DOWN:  // SwiGLU output -> down rows, residual add; split along K in 3 segments
-            if (!a.kpart || !a.kcnt) return hipErrorInvalidValue;
+            if (!a.kpart || !a.kcnt || a.N > a.krows) return hipErrorInvalidValue;
             return one ? launch_one<FMT, FF, 4, 1, PRO_F32, EPI_RESID>(a, H / 16 * (FF / SEG), s)
                        : launch_one<FMT, FF, 4, MAXM, PRO_F32, EPI_RESID>(a, H / 16 * (FF / SEG), s);
         case GEMV_LMHEAD:  // final RMSNorm -> tied embedding rows -> argmax partials

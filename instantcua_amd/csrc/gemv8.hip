@@ -543,10 +543,10 @@ template <int FMT, int K, int PRO, int EPI, int NR>
 static hipError_t launch(const GemvArgs& a, hipStream_t s) {
     const int nrb = EPI == EPI_SWIGLU ? FF / 8 : a.N / 16;
     if constexpr (K == FF && PRO == PRO_F32 && (EPI == EPI_RESID || EPI == EPI_STORE)) {
-        // With buffers of [3][MAXM][N] sums and N / 16 counters (the engine's, N = 2048; a standalone
-        // product's up to one row block a CU, where walking the three segments in one workgroup
-        // serialises three memory round trips).
-        if (a.kpart && a.kcnt) {
+        // Up to the rows that the partials hold (the engine's N = 2048; a standalone product's one row
+        // block a CU, up to which walking the three segments in one workgroup only serialises three
+        // memory round trips).
+        if (a.kpart && a.kcnt && a.N <= a.krows) {
             hipLaunchKernelGGL((gemv8_split_kernel<FMT, EPI, NR>), dim3(nrb * (K / SEG)), dim3(THREADS), 0, s, a);
             return hipGetLastError();
         }

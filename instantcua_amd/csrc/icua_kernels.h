@@ -38,6 +38,7 @@ struct GemvArgs {
     int blocks;             // isolated GEMV launches: grid size
     float* kpart;           // K = 6144 residual GEMV: per-segment partials [3][MAXM][N]
     int* kcnt;              // and per-row-block arrival counters [N / 16], zero between launches
+    int krows;              // the N that the two buffers hold
     uint8_t* apre;          // multi-row passes: operands pre-staged by launch_gemv_prep (or null)
     float* fxpre;           // and their group factors
 };

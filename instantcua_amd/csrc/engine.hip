@@ -929,7 +929,8 @@ struct icua_engine {
         for (int c0 = 0; c0 < n; c0 += PF_CHUNK) {
             M = std::min(PF_CHUNK, n - c0);
             const int parts = (flags & ICUA_FLAG_PREFILL_FP16) ? 1 : 2;
-            const int pad = pf_use_split(fmt, parts, M) && (parts == 2 || M <= 64) ? 64 : 128, Mpad = (M + pad - 1) / pad * pad;
+            const int pad = pf_use_split(fmt, parts, M) && (parts == 2 || M <= 64) ? 64 : 128;
+            const int Mpad = (M + pad - 1) / pad * pad;
             EmbedArgs ea{};
             ea.toks = prompt;
             ea.E = E;

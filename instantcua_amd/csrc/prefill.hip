@@ -386,9 +386,8 @@ __global__ __launch_bounds__(512) void pf_gemm_kernel(PfGemmArgs a) {
     const uint32_t* vsrc = (const uint32_t*)a.sb + (size_t)(tn * TR + (tid % TR)) * NG + (tid / TR);
     constexpr int vstride = 2;
     const bool vload = !DQ && (2 * TR >= 512 || tid < 2 * TR);
-    // DQ q4 / q8: the unpacking thread's own scale words, row (tn RB + srb + 8 hb) 16 + lane % 16,
-    // words 2 c and 2 c + 1 of step c (q4 the (scale, bias) of 64-groups 2 c, 2 c + 1; q8 the
-    // scales of 32-groups 4 c .. 4 c + 3).
+    // DQ q8: the unpacking thread's own scale words, row (tn RB + srb + 8 hb) 16 + lane % 16, words 2 c
+    // and 2 c + 1 of step c (the scales of 32-groups 4 c .. 4 c + 3).
     const uint32_t* dsrc = (const uint32_t*)a.sb + (size_t)((tn * PG_RB + srb) * 16 + (lane & 15)) * NG;
     constexpr size_t DSRC2 = (size_t)8 * 16 * NG;  // row block srb + 8
 
@@ -576,7 +575,7 @@ __global__ __launch_bounds__(512) void pf_gemm_kernel(PfGemmArgs a) {
     aload(0, Ae);
     aload(1, Ao);
     wload(0);
-    if constexpr (FMT == FMT_Q4 && !DQ) {
+    if constexpr (FMT == FMT_Q4) {
         // The q4 bias term sum_g b_g X_g of every output, on the matrix cores before the loop:
         // per 32 groups, A = the token block's group sums X (scaled by 2^-8 into fp16 range,
         // hi + lo parts) and B = the rows' fp16 biases, exact.  The loop's group epilogue is then
@@ -1071,10 +1070,6 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const uint16_t* kg = a.kc + (size_t)g * a.maxctx * HD;
     const uint16_t* vg = a.vc + (size_t)g * a.maxctx * HD;
 
-    // Staging of half hb: K key tid / 8, dims 16 (tid % 8) .. + 15; V keys 4 (tid / 32) .. + 3,
-    // dims 4 (tid % 32) .. + 3 (transposed in registers, 8-byte LDS writes).
-    uint4 kr0[2], kr1[2];
-    uint2 vr0[4], vr1[4];
     // Staging through buffer resources bounded at kv_lim: slots at or past it (masked for every
     // query of the block) read as zeros, with no branch.  Half hb of iteration it: K key tid / 8,
     // dims 16 (tid % 8) .. + 15; V keys 4 (tid / 32) .. + 3, dims 4 (tid % 32) .. + 3 (transposed
@@ -1437,7 +1432,10 @@ hipError_t launch_pf_gemm(int fmt, int K, int epi, const PfGemmArgs& a, hipStrea
     if (a.M < 1 || a.N % 256 || (a.parts != 1 && a.parts != 2) || a.splits < 1 || (a.splits > 1 && !a.part))
         return hipErrorInvalidValue;
     if (pf_use_split(fmt, a.parts, a.M)) {
-        if (a.splits != pf_gemm_splits(fmt, a.parts, K, a.N, a.M) || a.Mpad < (a.M + 63) / 64 * 64 || (a.parts == 1 && a.Mpad % 128 && a.M > 64)) return hipErrorInvalidValue;
+        // The tiles of 128 tokens (fp16 operands alone) need rows up to a multiple of 128.
+        const int pad = a.parts == 1 && a.M > 64 ? 128 : 64;
+        if (a.splits != pf_gemm_splits(fmt, a.parts, K, a.N, a.M) || a.Mpad < (a.M + pad - 1) / pad * pad)
+            return hipErrorInvalidValue;
         switch (fmt) {
             case FMT_Q4: return pf_split_fmt<FMT_Q4>(K, epi, a, s);
             case FMT_Q8: return pf_split_fmt<FMT_Q8>(K, epi, a, s);

@@ -1319,6 +1319,14 @@ int icua_generate_vision(icua_engine* e, const uint8_t* rgb, int width, int heig
     return 0;
 }
 
+// Whether host memory is pinned.
+static bool pinned(const void* p) {
+    hipPointerAttribute_t a{};
+    const bool known = hipPointerGetAttributes(&a, p) == hipSuccess;
+    if (!known) (void)hipGetLastError();  // ordinary memory is no error here
+    return known && a.type == hipMemoryTypeHost;
+}
+
 int icua_verify(icua_engine* e, const int32_t* draft, int m, int32_t* out_argmax, float* out_logits) {
     if (!e || !draft || !out_argmax) return fail("null argument");
     if (m < 1 || m > MAXM) return fail("verify takes 1..8 draft tokens");
@@ -1349,13 +1357,16 @@ int icua_verify(icua_engine* e, const int32_t* draft, int m, int32_t* out_argmax
         if (e->enqueue_layer(l, MAXM, 0, m)) return -1;
     if (e->enqueue_head(MAXM, 1, m)) return -1;
     if (e->write_state(s)) return -1;
+    // Logits go to pinned memory on the stream, behind one wait; to pageable memory by a plain copy
+    // after it, as there a copy on the stream takes up to 0.2 ms longer where pages are written for the
+    // first time (one row, 4 layers: 551 us a call against 313).
+    const size_t bytes = sizeof(float) * (size_t)m * VOCAB;
+    const bool async = out_logits && pinned(out_logits);
     HIPCK(hipMemcpyAsync(out_argmax, e->argmax_rows, sizeof(int32_t) * m, hipMemcpyDeviceToHost, e->stream));
+    if (async) HIPCK(hipMemcpyAsync(out_logits, e->logits, bytes, hipMemcpyDeviceToHost, e->stream));
     HIPCK(hipStreamSynchronize(e->stream));
     idle.done();
-    // Not on the stream: into pageable memory written for the first time such a copy took 0.2 ms longer
-    // (one row, 4 layers: 551 us a call against 313), and elsewhere it is no faster.
-    if (out_logits)
-        HIPCK(hipMemcpy(out_logits, e->logits, sizeof(float) * (size_t)m * VOCAB, hipMemcpyDeviceToHost));
+    if (out_logits && !async) HIPCK(hipMemcpy(out_logits, e->logits, bytes, hipMemcpyDeviceToHost));
     e->last_logits_rows = m;
     return 0;
 }

@@ -54,6 +54,7 @@ int hipGetDevice(int* d) { return *d = 0, OK; }
 int hipDeviceGetAttribute(int* v, int a, int d) { return (void)a, (void)d, *v = 0, OK; }
 int hipGetLastError(void) { int e = (int)last_error; return last_error = 0, e; }
 const char* hipGetErrorString(int e) { return e ? "failed on request" : "no error"; }
+int hipPointerGetAttributes(void* a, const void* p) { return (void)a, (void)p, last_error = 1; } /* no pinned memory */
 int hipFuncSetAttribute(const void* f, int a, int v) { return (void)f, (void)a, (void)v, OK; }
 int hipGetSymbolAddress(void** p, const void* s) { return *p = (void*)s, OK; }
 int hipStreamBeginCapture(void* s, int m) { return (void)s, (void)m, capturing = 1, OK; }

@@ -541,18 +541,19 @@ __global__ __launch_bounds__(256 * VA_PARTS) void vit_attention_kernel(const uin
     }
 }
 
-template <int PARTS>
-hipError_t attention_parts(const VitBuffers& b, int np, hipStream_t s) {
-    const hipError_t e = hipFuncSetAttribute((const void*)vit_attention_kernel<PARTS>,
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)va_lds_bytes(PARTS));
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(vit_attention_kernel<PARTS>, dim3((np + 63) / 64, VNH), dim3(256 * PARTS), va_lds_bytes(PARTS), s, b.q, b.k,
-                       b.vt, b.attn, np, NPATCH_MAX);
-    return hipGetLastError();
+int attention_parts(int np) { return np <= 640 ? 2 : 4; }
+
+hipError_t attention_setup(int np) {
+    const int parts = attention_parts(np);
+    return hipFuncSetAttribute(parts == 2 ? (const void*)vit_attention_kernel<2> : (const void*)vit_attention_kernel<4>,
+                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)va_lds_bytes(parts));
 }
 
 hipError_t attention(const VitBuffers& b, int np, hipStream_t s) {
-    return np <= 640 ? attention_parts<2>(b, np, s) : attention_parts<4>(b, np, s);
+    const int parts = attention_parts(np);
+    hipLaunchKernelGGL(parts == 2 ? vit_attention_kernel<2> : vit_attention_kernel<4>, dim3((np + 63) / 64, VNH),
+                       dim3(256 * parts), va_lds_bytes(parts), s, b.q, b.k, b.vt, b.attn, np, NPATCH_MAX);
+    return hipGetLastError();
 }
 
 template <int BN, int BM, int WN, int WM, int MODE, int S>
@@ -617,6 +618,7 @@ hipError_t merger(const VitMerger& mg, const uint16_t* xn, int nvis, uint16_t* h
 hipError_t launch_vision(const VitWeights& w, const VitBuffers& b, int gh, int gw, hipStream_t s) {
     const int np = gh * gw, nvis = np / 4;
     if (gh < 2 || gw < 2 || gh % 2 || gw % 2 || np > NPATCH_MAX) return hipErrorInvalidValue;
+    VCK(attention_setup(np));
     hipLaunchKernelGGL(vit_patchify_kernel, dim3(np), dim3(256), 0, s, b.rgb, b.patches, gh, gw);
     VCK(hipGetLastError());
     VitGemmArgs g{};
